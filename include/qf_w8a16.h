@@ -317,6 +317,13 @@ int qf_w8a8_launch_plan(int M, int N, int K, int layout, const qf_w8a16_config* 
 int qf_quantize_rows_int8(const uint16_t* w, int64_t ldw, int8_t* q, float* s,
                           int V, int H, void* stream);
 
+/* qf_quantize_rows_int8 followed by qf_w8a16_repack in one pass: the same scales, and the TILED image
+ * (qf_w8a16_tiled_bytes(V, H) bytes, pad rows 0) of the same int8 rows.  H % 64 == 0, H <= 18432, w and
+ * image 16-byte aligned, ldw % 8 == 0, else QF_ERR_UNSUPPORTED (the caller then makes the two calls).
+ * Reference: plugin/qwen_fastpath/patches.py:139-147 (the quantiser; the image is this library's own). */
+int qf_quantize_rows_int8_tiled(const uint16_t* w, int64_t ldw, int8_t* image, float* s, int V, int H,
+                                void* stream);
+
 /* Row argmax of bf16 logits [M, N] (row stride ld): columns >= n_valid count as -inf (the padded
  * vocabulary), ties go to the lowest index, NaN counts as the maximum (torch.argmax semantics).
  * out[m] = index + index_offset (int64).  Reference: plugin/qwen_fastpath/patches.py:182-185. */

@@ -1271,19 +1271,49 @@ __device__ __forceinline__ float quant_amax8(float amax, const u32x4_t v) {
   return amax;
 }
 
-__device__ __forceinline__ u32x2_t quant_pack8(const u32x4_t v, float s) {
+// A row's int8 scale s with its rounded reciprocal.  `plain`: s is far from fp32's underflow and overflow ends,
+// and the quotient x / s of a bf16 x takes a multiply and two fused multiply-adds (one step of the residual
+// correction that Markstein's division theorem is built on, IBM J. Res. Dev. 34 (1990)) instead of the dozen
+// instructions of an IEEE division.  The step gives the IEEE quotient itself for every value that can meet a scale
+// here: s is fl(1/127) times a bf16 maximum (or the 1e-8 floor) and x a bf16 no larger, so apart from a power of two
+// there are 129 x 128 pairs, and tests/test_oracle.py compares all of them.  Rows outside the range (a maximum
+// below 2^-60, an infinity) divide.
+struct QuantScale {
+  float s, r;
+  bool plain;
+};
+__device__ __forceinline__ QuantScale quant_scale(float s) {
+  QuantScale q;
+  q.s = s;
+  q.r = __fdiv_rn(1.0f, s);
+  q.plain = s >= 0x1p-67f && s <= 0x1.fffffep+127f;
+  return q;
+}
+
+// 8 bf16 values of a row -> 8 int8: rint(x / s) (half to even) clamped to [LO, 127], NaN going to LO, and 0 for every
+// value of a row whose scale is 0.  Adding 1.5 * 2^23 rounds a value of at most 128 in magnitude half to even and
+// leaves the integer in the low bits of the sum.
+template <int LO, bool PLAIN>
+__device__ __forceinline__ u32x2_t quant_pack8(const u32x4_t v, const QuantScale q) {
   uint32_t b[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    const float f = __uint_as_float((i & 1) ? (v[i >> 1] & 0xffff0000u) : (v[i >> 1] << 16));
-    float t = s > 0.f ? rintf(__fdiv_rn(f, s)) : 0.f;
-    t = fminf(fmaxf(t, -128.f), 127.f);
-    b[i] = (uint32_t)(int)t & 0xffu;
+    const float x = __uint_as_float((i & 1) ? (v[i >> 1] & 0xffff0000u) : (v[i >> 1] << 16));
+    float t;
+    if constexpr (PLAIN) {
+      const float q0 = x * q.r;
+      t = __builtin_fmaf(__builtin_fmaf(-q0, q.s, x), q.r, q0);
+    } else {
+      t = q.s > 0.f ? __fdiv_rn(x, q.s) : 0.f;
+    }
+    b[i] = __float_as_uint(__builtin_amdgcn_fmed3f(t, (float)LO, 127.f) + 0x1.8p+23f);
   }
-  u32x2_t o;
-  o.x = b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24);
-  o.y = b[4] | (b[5] << 8) | (b[6] << 16) | (b[7] << 24);
-  return o;
+  // the low bytes of four words
+  auto low4 = [](uint32_t b0, uint32_t b1, uint32_t b2, uint32_t b3) {
+    return __builtin_amdgcn_perm(__builtin_amdgcn_perm(b3, b2, 0x0c0c0400u), __builtin_amdgcn_perm(b1, b0, 0x0c0c0400u),
+                                 0x05040100u);
+  };
+  return u32x2_t{low4(b[0], b[1], b[2], b[3]), low4(b[4], b[5], b[6], b[7])};
 }
 
 // With tiled != 0 the int8 row goes to the token-tiled image instead of a row of xq (8 values of row m
@@ -1331,7 +1361,9 @@ __global__ void __launch_bounds__(256) quantize_tokens_kernel(const uint16_t* x,
   const float inv127 = 1.0f / 127.0f;  // constant-folded: the fp32 reciprocal of 127
   const float s = amax * inv127;
   if (threadIdx.x == 0) s_a[m] = s;
+  const QuantScale qs = quant_scale(s);  // the row's, so uniform
   const int ksteps = K / kStepK;
+  auto pack = [&](const u32x4_t v) { return qs.plain ? quant_pack8<-128, true>(v, qs) : quant_pack8<-128, false>(v, qs); };
   auto dst = [&](int c) -> u32x2_t* {
     return reinterpret_cast<u32x2_t*>(tiled ? xq + token_tile_offset(m, 8 * c, ksteps) : xq + m * ldq + 8 * c);
   };
@@ -1339,11 +1371,93 @@ __global__ void __launch_bounds__(256) quantize_tokens_kernel(const uint16_t* x,
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
       const int c = (int)threadIdx.x + i * 256;
-      if (c < pieces) *dst(c) = quant_pack8(keep[i], s);
+      if (c < pieces) *dst(c) = pack(keep[i]);
     }
   } else {
-    for (int c = threadIdx.x; c < pieces; c += 256) *dst(c) = quant_pack8(row[c], s);
+    for (int c = threadIdx.x; c < pieces; c += 256) *dst(c) = pack(row[c]);
   }
+}
+
+// Per-row quantiser straight into the TILED image (HEAD: the draft head's rows, s = max(amax, 1e-8) fl(1/127),
+// clamp +-127; else tokens, s = amax fl(1/127), clamp [-128, 127]).  A workgroup of W wavefronts takes R rows of one
+// 16-row tile: lane (c, r) of a wavefront holds 16 consecutive values of row r (two 16-byte loads), which are exactly
+// one 16-byte piece of the image, and the R pieces at one k lie side by side there, so every store instruction writes
+// 64 / R segments of 16 R contiguous bytes (R = 16: one whole KiB, R = 8: whole 128-byte lines) and no line is put
+// together from several workgroups.  The row's values stay in registers between the maximum and the rounding (NP
+// piece pairs a lane).  Memory-bound: tokens
+// 4096 x 5120 / 8192 / 17408 (x rotating past the last-level cache) 14.5 / 22.0 / 53.1 us against 18.1 / 29.1 / 55.6
+// for a workgroup a row; the 151936 x 5120 head 411 us (5.7 TB/s) against 443 + 272 us for the quantiser and the
+// repack.  W = 16, R = 16 and R = 4 at K = 5120: 15.2 to 16.7 us, the head 423 to 483 us.  Non-temporal token loads
+// are 3% faster, non-temporal stores 5% more here, but the GEMM that reads the image then loses it (level together).
+template <int R, int W, int NP, bool HEAD>
+__global__ void __launch_bounds__(W * kWave) quantize_tiled_kernel(const uint16_t* x, int64_t ldx, int K, int8_t* image,
+                                                                   float* scale, int M) {
+  constexpr int C = kWave / R;  // 16-value pieces of a row a wavefront takes at once
+  constexpr int LO = HEAD ? -127 : -128;
+  __shared__ float red[W][R];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = threadIdx.x / kWave;
+  const int r = lane % R, c0 = wave * C + lane / R;
+  const int pieces = K / 16;
+  const int64_t m = (int64_t)blockIdx.x * R + r;
+  const u32x4_t* row = reinterpret_cast<const u32x4_t*>(x + min(m, (int64_t)M - 1) * ldx);  // rows past M: written as 0
+  float amax = 0.f;
+  u32x4_t keep[2 * NP];
+  auto load = [&](int i) {
+    return HEAD ? row[i] : load16<true>(reinterpret_cast<const int8_t*>(row + i));
+  };
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    const int c = c0 + i * W * C;
+    const bool in = c < pieces;
+    keep[2 * i] = in ? load(2 * c) : (u32x4_t){0u, 0u, 0u, 0u};
+    keep[2 * i + 1] = in ? load(2 * c + 1) : (u32x4_t){0u, 0u, 0u, 0u};
+  }
+#pragma unroll
+  for (int i = 0; i < 2 * NP; ++i) amax = quant_amax8(amax, keep[i]);
+#pragma unroll
+  for (int off = R; off < kWave; off *= 2) amax = fmaxf(amax, __shfl_xor(amax, off, kWave));
+  if (lane < R) red[wave][lane] = amax;
+  __syncthreads();
+  amax = red[0][r];
+#pragma unroll
+  for (int i = 1; i < W; ++i) amax = fmaxf(amax, red[i][r]);
+  const float inv127 = 1.0f / 127.0f;  // constant-folded: the fp32 reciprocal of 127
+  const QuantScale qs = quant_scale((HEAD ? fmaxf(amax, 1e-8f) : amax) * inv127);
+  if (wave == 0 && lane < R && m < M) scale[m] = qs.s;
+  // piece c of the row at byte (tile * K / 64 + c / 4) * 1024 + 256 (c % 4) + 16 (m % 16) = tile * 16 K + 256 c + ...
+  u32x4_t* out = reinterpret_cast<u32x4_t*>(image + (m >> 4) * 16 * (int64_t)K + 16 * (m & 15));
+  const bool plain = __all(qs.plain);
+  auto store = [&](int c, const u32x4_t a, const u32x4_t b) {
+    const u32x2_t lo = plain ? quant_pack8<LO, true>(a, qs) : quant_pack8<LO, false>(a, qs);
+    const u32x2_t hi = plain ? quant_pack8<LO, true>(b, qs) : quant_pack8<LO, false>(b, qs);
+    const u32x4_t v = m < M ? u32x4_t{lo.x, lo.y, hi.x, hi.y} : u32x4_t{0u, 0u, 0u, 0u};
+    if (c < pieces) {
+      out[16 * (int64_t)c] = v;
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < NP; ++i) store(c0 + i * W * C, keep[2 * i], keep[2 * i + 1]);
+}
+
+// The workgroup shape for rows of K values, by the registers a row takes: 8 wavefronts, 8 rows a workgroup up to
+// K = 8192, 4 rows up to kQuantTiledMaxK (R = 8 would keep 72 or more registers of the row a lane; R = 4 stores
+// segments of 64 bytes; K = 17408: 53.1 us, R = 8 over 100).
+constexpr int kQuantTiledMaxK = 18432;
+constexpr int kQuantTiledMinRows = 1024;
+template <bool HEAD>
+hipError_t launch_quantize_tiled(const uint16_t* x, int64_t ldx, int M, int K, int8_t* image, float* scale,
+                                 hipStream_t st) {
+  const int rows = (M + 15) / 16 * 16;
+  constexpr int W = 8;
+  const dim3 block(W * kWave);
+  if (K <= 5120)
+    hipLaunchKernelGGL((quantize_tiled_kernel<8, W, 5, HEAD>), dim3(rows / 8), block, 0, st, x, ldx, K, image, scale, M);
+  else if (K <= 8192)
+    hipLaunchKernelGGL((quantize_tiled_kernel<8, W, 8, HEAD>), dim3(rows / 8), block, 0, st, x, ldx, K, image, scale, M);
+  else
+    hipLaunchKernelGGL((quantize_tiled_kernel<4, W, 9, HEAD>), dim3(rows / 4), block, 0, st, x, ldx, K, image, scale, M);
+  return hipGetLastError();
 }
 
 typedef int32_t i32x4_t __attribute__((ext_vector_type(4)));
@@ -3740,12 +3854,26 @@ int qf_quantize_rows_int8(const uint16_t* w, int64_t ldw, int8_t* q, float* s, i
   return hipGetLastError() == hipSuccess ? QF_OK : QF_ERR_HIP;
 }
 
+int qf_quantize_rows_int8_tiled(const uint16_t* w, int64_t ldw, int8_t* image, float* s, int V, int H, void* stream) {
+  if (w == nullptr || image == nullptr || s == nullptr || V < 1 || H < 1 || ldw < H) return QF_ERR_INVALID_ARG;
+  if (H % QF_W8A16_K_ALIGN || H > kQuantTiledMaxK || !aligned16(w) || ldw % 8 || !aligned16(image))
+    return QF_ERR_UNSUPPORTED;
+  return launch_quantize_tiled<true>(w, ldw, V, H, image, s, reinterpret_cast<hipStream_t>(stream)) == hipSuccess
+             ? QF_OK
+             : QF_ERR_HIP;
+}
+
 static int quantize_tokens(const uint16_t* x, int64_t ldx, int M, int K, int8_t* xq, int64_t ldq, float* s_a,
                            int tiled, void* stream) {
   if (x == nullptr || xq == nullptr || s_a == nullptr || M < 1 || K < 1 || ldx < K || ldq < K) return QF_ERR_INVALID_ARG;
   if (K % QF_W8A16_K_ALIGN || !aligned16(x) || ldx % 8 || (uintptr_t)xq % 8 || ldq % 8) return QF_ERR_UNSUPPORTED;
   if (tiled && !aligned16(xq)) return QF_ERR_UNSUPPORTED;
   const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  // Many rows: several rows of a tile a workgroup (whole lines stored); few: a workgroup a row, which
+  // puts more of them in flight (us, new against old: M = 333 4.6 / 4.1 at K = 5120 and 8.4 / 7.3 at 17408, M = 1024
+  // 5.6 / 5.6 and 13.4 / 17.4, M = 2048 8.3 / 11.3 and 26.1 / 29.7).
+  if (tiled && M >= kQuantTiledMinRows && K <= kQuantTiledMaxK)
+    return launch_quantize_tiled<false>(x, ldx, M, K, xq, s_a, st) == hipSuccess ? QF_OK : QF_ERR_HIP;
   const int per_thread = ceil_div(K / 8, 256);  // 16-byte pieces a thread
   const dim3 grid(tiled ? round_up16(M) : M);
   if (per_thread <= 4)

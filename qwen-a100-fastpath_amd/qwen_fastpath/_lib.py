@@ -54,6 +54,7 @@ EXPORTS = (
     "qf_rms_norm_rows_bf16",
     "qf_w8a16_gemm_rmsnorm",
     "qf_quantize_rows_int8",
+    "qf_quantize_rows_int8_tiled",
     "qf_argmax_rows_bf16",
     "qf_argmax_rows_workspace_bytes",
     "qf_argmax_rows_bf16_ws",
@@ -154,6 +155,8 @@ def load() -> ctypes.CDLL:
     L.qf_w8a16_gemm_rmsnorm.restype = i32
     L.qf_quantize_rows_int8.argtypes = [p, i64, p, p, i32, i32, p]
     L.qf_quantize_rows_int8.restype = i32
+    L.qf_quantize_rows_int8_tiled.argtypes = [p, i64, p, p, i32, i32, p]
+    L.qf_quantize_rows_int8_tiled.restype = i32
     L.qf_argmax_rows_bf16.argtypes = [p, i64, i32, i32, i32, i64, p, p]
     L.qf_argmax_rows_bf16.restype = i32
     L.qf_argmax_rows_workspace_bytes.argtypes = []

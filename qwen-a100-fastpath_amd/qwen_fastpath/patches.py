@@ -28,7 +28,7 @@ from typing import Callable, NamedTuple, Optional
 import torch
 
 from . import _lib as L
-from .w8a16 import (ROWMAJOR, SMALL_M, TILED, _workspace, from_tiled, pick_config, to_tiled, w8a16_mm,
+from .w8a16 import (ROWMAJOR, SMALL_M, TILED, _workspace, from_tiled, pick_config, tiled_numel, to_tiled, w8a16_mm,
                     w8a16_mm_argmax, w8a16_mm_prefill, w8a8_mm)
 
 logger = logging.getLogger("vllm.qwen_fastpath")
@@ -572,10 +572,31 @@ def quantize_lm_head(weight: torch.Tensor):
     return w8, scale
 
 
+def _quantize_lm_head_tiled(weight: torch.Tensor):
+    """quantize_lm_head's int8 rows as their TILED image, with the scales, in one pass over the bf16 head
+    (qf_quantize_rows_int8_tiled); None where that pass does not serve the head."""
+    if weight.dtype != torch.bfloat16 or weight.dim() != 2 or not weight.is_cuda or weight.stride(1) != 1:
+        return None
+    V, H = weight.shape
+    img = torch.empty(tiled_numel(V, H), dtype=torch.int8, device=weight.device)
+    scale = torch.empty((V,), dtype=torch.float32, device=weight.device)
+    stream = torch.cuda.current_stream(weight.device).cuda_stream
+    rc = L.load().qf_quantize_rows_int8_tiled(weight.data_ptr(), weight.stride(0), img.data_ptr(), scale.data_ptr(),
+                                              V, H, stream)
+    if rc == L.ERR_UNSUPPORTED:
+        return None
+    L.check(rc, "qf_quantize_rows_int8_tiled")
+    return img, scale
+
+
 def make_int8_head(weight: torch.Tensor, num_pad: int = 0, layout: int = TILED) -> Int8Head:
     """The draft head's int8 copy.  The copy is this plugin's own (the checkpoint's bf16 head is left
     as it is), so it is kept in the TILED layout the kernel streams fastest; layout=ROWMAJOR keeps the
     reference's [V, H] row-major copy (patches.py:149)."""
+    if layout == TILED:
+        tiled = _quantize_lm_head_tiled(weight)
+        if tiled is not None:
+            return Int8Head(*tiled, int(num_pad), pick_config(*weight.shape, TILED), TILED)
     w8, scale = quantize_lm_head(weight)
     V, H = w8.shape
     cfg = pick_config(V, H, layout)

@@ -148,6 +148,26 @@ def test_quantizer_kernels_bit_exact(oracle, H):
     assert np.array_equal(w8.cpu().numpy(), q_ref)
 
 
+@pytest.mark.parametrize("V,H", [(1, 64), (15, 5120), (16, 5184), (257, 8192), (33, 8256), (40, 18432), (40, 18496)])
+def test_quantise_to_image_equals_two_passes(V, H):
+    """make_int8_head's one-pass image and scales against the row-major quantiser and the repack, byte for byte, at
+    the edges of the row shapes (5120, 8192, 18432; 18496 takes the two passes): zero, tiny, huge and infinite rows,
+    NaN values, a strided head, pad rows."""
+    g = torch.Generator(device=DEV).manual_seed(V * 7 + H)
+    w = torch.randn(V, H + 8, device=DEV, generator=g)
+    w = (w * torch.exp2(torch.randint(-30, 30, (V, 1), device=DEV, generator=g).float())).to(torch.bfloat16)[:, :H]
+    for i, v in enumerate((0.0, 1e-30, 3e38, float("inf"))):
+        if V > 4 * i + 4:
+            w[4 * i, :] = 0
+            w[4 * i, 5:60] = v
+    w[V // 2, 3] = float("nan")
+    head = qf.make_int8_head(w)
+    w8, scale = qf.quantize_lm_head(w)
+    torch.cuda.synchronize()
+    assert head.layout == qf.TILED and torch.equal(head.scale, scale)
+    assert torch.equal(head.w_t, qf.to_tiled(w8.t()))
+
+
 def test_draft_head_logits_and_argmax(oracle):
     """int8 draft logits through the W8A16 kernel (patches.py:157-166) and the pad-masked argmax
     (patches.py:182-185), against the oracle.  A row whose top-2 exact logits are within 2 bf16 ulp

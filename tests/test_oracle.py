@@ -389,3 +389,23 @@ def test_w8a8_oracle_rejects_planted_mistakes(oracle):
     col = (np.abs(xf).max(axis=0).astype(np.float32) * np.float32(1 / 127)).astype(np.float32)
     assert not np.allclose(run(np.full(8, col.mean(), np.float32), np.clip(np.rint(xf / col[None, :]), -128, 127)),
                            y, rtol=1e-3)
+
+
+def test_quantiser_quotient_equals_ieee_division():
+    """The kernels' quotient of a bf16 value by a row's scale, q0 = x r, q = fma(fma(-q0, s, x), r, q0) with r the
+    rounded 1 / s, equals the IEEE fp32 quotient for every pair that can meet, up to a power of two: s = fl(1/127)
+    times a bf16 maximum (128 significands) or the 1e-8 floor, x a bf16 value no larger (128 significands, 40
+    exponents: far below half a step).  The fused steps are exact in fp64 before their one rounding: q0 s and
+    x - q0 s need at most 48 bits, and the last sum's double rounding would only show as a mismatch."""
+    f = np.float32
+    sig = f(1) + np.arange(128, dtype=f) / f(128)
+    xs = np.concatenate([sig * f(2.0) ** -k for k in range(40)]).astype(f)
+    inv127 = f(1) / f(127)
+    for amax, top in [(a, f(1)) for a in sig] + [(f(1e-8), f(2.0) ** -27)]:
+        s = f(amax * inv127)
+        x = (xs * top)[xs * top <= amax]
+        r = f(1) / s
+        q0 = (x * r).astype(f)
+        e = (x.astype(np.float64) - q0.astype(np.float64) * np.float64(s)).astype(f)
+        q = (q0.astype(np.float64) + e.astype(np.float64) * np.float64(r)).astype(f)
+        assert np.array_equal(q, (x / s).astype(f)), amax

@@ -54,6 +54,8 @@ extern "C" {
 #define QF_SPEC_ATTN_MIN_PAGE 16
 /* Prefix splits are whole multiples of this many positions (the prefix kernel's key block). */
 #define QF_SPEC_ATTN_KEY_BLOCK 32
+/* Bytes a balanced call's workspace holds besides the partials (each request's place among the splits). */
+#define QF_SPEC_ATTN_PLAN_BYTES 512
 
 /* ABI version of the loaded library (QF_SPEC_ATTN_ABI_VERSION). */
 int qf_spec_attn_abi_version(void);
@@ -81,6 +83,25 @@ int qf_spec_attention(const uint16_t* query, int64_t q_stride_tok, int64_t q_str
                       int num_reqs, int q_len, int num_heads, int num_kv_heads, int head_size,
                       int page_size, float scale, int num_splits, int min_chunk,
                       void* workspace, size_t workspace_bytes, void* stream);
+
+/* qf_spec_attention with one set of split slots per kv head shared by all requests: total_splits slots
+ * (num_reqs <= total_splits <= 65535, num_reqs <= 64, else QF_ERR_UNSUPPORTED) are given out by length, one
+ * chunk length for the whole batch (at least min_chunk, a multiple of QF_SPEC_ATTN_KEY_BLOCK), so a ragged
+ * batch's longest split is about its mean.  Workspace: qf_spec_attn_workspace_bytes(1, q_len, num_heads,
+ * num_kv_heads, head_size, total_splits) + QF_SPEC_ATTN_PLAN_BYTES.  The rest as qf_spec_attention; the results differ by the order of
+ * the fp32 sums only.  No reference counterpart (the reference splits every request num_splits ways,
+ * plugin/qwen_fastpath/spec_attn.py:38-40). */
+int qf_spec_attention_balanced(const uint16_t* query, int64_t q_stride_tok, int64_t q_stride_head,
+                               const uint16_t* key_cache, int64_t k_stride_block, int64_t k_stride_tok,
+                               int64_t k_stride_head,
+                               const uint16_t* value_cache, int64_t v_stride_block, int64_t v_stride_tok,
+                               int64_t v_stride_head,
+                               const int32_t* block_table, int64_t bt_stride,
+                               const int32_t* seq_lens,
+                               uint16_t* out, int64_t o_stride_tok, int64_t o_stride_head,
+                               int num_reqs, int q_len, int num_heads, int num_kv_heads, int head_size,
+                               int page_size, float scale, int total_splits, int min_chunk,
+                               void* workspace, size_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }

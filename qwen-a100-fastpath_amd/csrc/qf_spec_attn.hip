@@ -7,22 +7,29 @@
 // q_len * G query rows sharing it; a second kernel attends this step's q_len positions causally and
 // merges everything by log-sum-exp.  The kernels themselves are designed for CDNA4:
 //
-//   prefix kernel, one 256-thread workgroup per (split, request, kv head); the last active split also
-//   takes this step's q_len in-flight positions, masked causally per query row:
-//   * K and V rows of a 32-position stage are copied global -> LDS with 16-byte direct-to-LDS loads
-//     (no VGPR staging), 16-byte pieces XOR-swizzled per row so that the MFMA fragment reads below
-//     are free of bank conflicts; a ring of kRing stages keeps kRing - 1 stages in flight while a
-//     stage is computed, with one barrier per stage.
-//   * Wavefront w takes key tile w & 1 (16 of the stage's 32 positions) and d half w >> 1.
-//   * S^T = K . Q^T on v_mfma_f32_16x16x32_bf16 with K as the A operand (16 positions x 32 d) and the
-//     packed query rows as B (16 rows), so each lane's accumulator holds 4 positions of ONE row: the
-//     online softmax needs only two cross-lane steps per row, and the lane's 4 probabilities are
-//     already its B fragment of the next product.
-//   * O^T = V^T . P^T on v_mfma_f32_16x16x16_bf16 over the tile's 16 positions and the wavefront's
-//     half of the head dimension; each V^T fragment is one transposing LDS read (ds_read_b64_tr_b16)
-//     of the row-major V rows.
-//   * The two key tiles keep separate softmax states (the two wavefronts of a d half compute the same
-//     scores), merged once per split through LDS; wavefronts never exchange state inside the loop.
+//   prefix kernel, one workgroup of 4 or 8 wavefronts per (split, kv head, request); the last active split also takes
+//   this step's q_len in-flight positions, masked causally per query row:
+//   * A stage is one 16-position key tile a wavefront.  Each wavefront copies its tile's K and V rows global -> LDS with
+//     16-byte direct-to-LDS loads (no VGPR staging), 16-byte pieces XOR-swizzled per row so that the MFMA fragment reads
+//     below are free of bank conflicts, into two slots of its own per tensor: the K of the stage after next and the V of
+//     the next stage are in flight while a stage is computed (64 KiB a workgroup at D = 256).
+//   * S^T = K . Q^T on v_mfma_f32_16x16x32_bf16 with K as the A operand (16 positions x 32 d) and the packed query rows
+//     as B (16 rows), each wavefront its own key tile and every row: no score is computed twice.  A lane's accumulator
+//     holds 4 positions of ONE row.
+//   * The softmax weights (rounded to bf16) meet in LDS, and each wavefront multiplies its own share of the head
+//     dimension for the whole stage: O^T = V^T . P^T on v_mfma_f32_16x16x32_bf16 over two key tiles at once, each V^T
+//     fragment two transposing LDS reads (ds_read_b64_tr_b16) of the row-major V rows.  So the accumulators are an
+//     eighth or a quarter of the output a wavefront, nothing is merged at the end but the rows' sums, and a stage costs
+//     one barrier.
+//   * The exponent reference of a row is shared by the wavefronts and moves only when a score exceeds it by 2^8; a stage
+//     in which one does is seen by all of them after its barrier and weighed again against the new references.
+//   What bounds it: memory at long contexts (38000 positions, D = 256, 4 kv heads: 30.2 us, 5.2 TB/s of K and V), the
+//   chain of dependent latencies at short ones (1000 positions: 7.7 us, of which the launch 1.7, sequence length ->
+//   block ids -> K and V about 3.5).  Against the form before it (4 wavefronts in two halves of the head dimension, each
+//   half computing every score, 32-position stages, a register state of the whole output merged through LDS), with its
+//   combine launch, us a layer: 38000 positions 40.1 -> 35.0; 1000 12.0 -> 10.8; D = 128, 30000 positions, 64 packed
+//   rows 55.0 -> 33.8; D = 64, four requests of 5000 18.3 -> 14.3.  Per-wavefront accumulators of the whole head
+//   dimension without a barrier in the loop measured 37.1 and 12.9 on the first two: their merge alone took 2.4 us.
 //   combine kernel, one 256-thread workgroup per (token, head, 64 d values): the row's split partials
 //   are merged by log-sum-exp in thread groups, then the groups through LDS.
 #include <hip/hip_runtime.h>
@@ -37,6 +44,8 @@ namespace qfa {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
@@ -45,14 +54,31 @@ typedef const void __attribute__((address_space(1)))* gptr_t;
 typedef void __attribute__((address_space(3)))* lptr_t;
 
 constexpr int kWave = 64;
-constexpr int kWaves = 4;
-constexpr int kThreads = kWave * kWaves;
-constexpr int kKeyBlock = QF_SPEC_ATTN_KEY_BLOCK;  // positions per stage
+constexpr int kThreads = 256;                      // combine kernel
+constexpr int kKeyBlock = QF_SPEC_ATTN_KEY_BLOCK;  // splits are whole multiples of this many positions
+constexpr int kMaxBalanced = kWave;                // requests of a balanced call: one lane of a wavefront each
+constexpr size_t kMaxLds = 160 * 1024;             // gfx950 LDS per workgroup
+static_assert(kMaxBalanced * sizeof(int2) <= QF_SPEC_ATTN_PLAN_BYTES, "a slot range a request");
 constexpr int kMaxRows = QF_SPEC_ATTN_MAX_ROWS;
-constexpr int kTablePages = 1024;  // block-table entries a prefix workgroup holds in LDS at once
+constexpr int kNonTemporal = 2;  // cache-policy operand of a direct-to-LDS load: read once
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr size_t kMaxDynLds = 160 * 1024 - 8 * 1024;  // gfx950 LDS per workgroup, less the static arrays
 constexpr size_t kDefaultLds = 64 * 1024;
+
+// Division of 0 <= n < 2^31 by an invariant d >= 1 (Granlund and Montgomery, PLDI 1994): with l = ceil(log2 d) and
+// m = ceil(2^(31 + l) / d), which has 32 bits, floor(n / d) = (n * m) >> (31 + l).
+struct Divisor {
+  uint32_t m;
+  int shift;  // of the upper half of the product; l = 0 (d = 1) is handled as m = 2^31, shift -1
+};
+inline Divisor divisor(int d) {
+  int l = 0;
+  while (((int64_t)1 << l) < d) ++l;
+  return Divisor{(uint32_t)((((uint64_t)1 << (31 + l)) + d - 1) / d), l - 1};
+}
+__device__ __forceinline__ int divide(int n, Divisor d) {
+  return (int)((((uint64_t)(uint32_t)n * d.m) >> 31) >> (d.shift + 1));
+}
 
 struct AttnArgs {
   const uint16_t* q;
@@ -66,27 +92,55 @@ struct AttnArgs {
   const int32_t* seq_lens;
   uint16_t* out;
   int64_t so_t, so_h;
-  float* o_part;    // [B][HKV][S][R][D]
-  float* lse_part;  // [B][HKV][S][R]
+  float* o_part;    // [B][HKV][S][R][D]; balanced: [HKV][S][R][D], request b's splits at its slots
+  float* lse_part;  // [B][HKV][S][R]; balanced: [HKV][S][R]
   int B, Q, H, HKV, G, R, page, splits, min_chunk;
+  // Not null: balanced.  The splits of a kv head are shared out over the requests by length; the prefix kernel leaves
+  // request b's first slot and slot count here for the combine kernel.
+  int2* plan;
+  Divisor by_g, by_splits, by_page;
   float qk_scale;  // softmax scale * log2(e): scores are kept in base 2
 };
 
 // Positions per prefix split (the reference's split arithmetic, spec_attn.py:38-40, with this
 // kernel's key block): both kernels derive it from the sequence length alone.
-__device__ __forceinline__ int split_chunk(int prefix, int splits, int min_chunk) {
-  int c = (prefix + splits - 1) / splits;
-  c = c > min_chunk ? c : min_chunk;
+__device__ __forceinline__ int split_chunk(int prefix, const AttnArgs& a) {
+  int c = prefix > 0 ? divide(prefix - 1, a.by_splits) + 1 : 0;
+  c = c > a.min_chunk ? c : a.min_chunk;
   return (c + kKeyBlock - 1) / kKeyBlock * kKeyBlock;
 }
 
-// Workgroup barrier for the copy ring.  Each wavefront has already waited for its own copies of the
-// stage (wait_vmcnt); no release fence is used, because at workgroup scope it would also wait for
-// the copies of later stages, which are LDS writes still in flight.  The acquire fence keeps the
-// stage's LDS reads (and the next copies into the ring) after the barrier.
-__device__ __forceinline__ void ring_barrier() {
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+// Inclusive scan over the wavefront's 64 lanes by DPP adds (every lane active).
+__device__ __forceinline__ int wave_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8: within 16 lanes
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast 15: row 0 into 1, row 2 into 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast 31: rows 0, 1 into 2, 3
+  return v;
+}
+
+// The balanced split (every lane of the wavefront active; at most kMaxBalanced requests, splits >= requests): one
+// chunk length for all requests, the shortest of a rising sequence of multiples of kKeyBlock whose splits fit the
+// a.splits slots of a kv head, so the longest split of a ragged batch is about the batch's mean and not the longest
+// request's share.  A request without a prefix takes one split (its in-flight positions).  Slots go to the requests
+// in order.  Lane i returns request i's length, splits (n) and first slot; `total` slots are used.
+__device__ __forceinline__ void balance(const AttnArgs& a, int lane, int& seq, int& chunk, int& n, int& first, int& total) {
+  seq = lane < a.B ? a.seq_lens[lane] : 0;
+  const int prefix = max(seq - a.Q, 0);
+  // total positions: at most 64 requests of below 2^31, in units of kKeyBlock so that the sum fits
+  const int units = __builtin_amdgcn_readlane(wave_scan((prefix + kKeyBlock - 1) / kKeyBlock), kWave - 1);
+  const int lo = max((units + a.splits - 1) / a.splits, (a.min_chunk + kKeyBlock - 1) / kKeyBlock);
+  chunk = lo * kKeyBlock;
+  for (;;) {  // ends: once chunk covers the longest prefix, every request takes one split and a.B <= a.splits
+    n = lane < a.B ? max((prefix + chunk - 1) / chunk, 1) : 0;
+    const int upto = wave_scan(n);
+    first = upto - n;
+    total = __builtin_amdgcn_readlane(upto, kWave - 1);
+    if (total <= a.splits) break;
+    chunk += (chunk / 8 + kKeyBlock - 1) / kKeyBlock * kKeyBlock;
+  }
 }
 
 // s_waitcnt with vmcnt = n (0..63) and the other counters unconstrained.
@@ -113,19 +167,65 @@ __device__ __forceinline__ u32x2_t ds_read_tr16_b64(uint32_t addr) {
   return v;
 }
 
-// Waits for every outstanding LDS read of the wavefront; the N fragments are tied to the wait, so no
-// use of them is scheduled before it.
-template <int N>
-__device__ __forceinline__ void wait_lds_all(u32x2_t (&v)[N]) {
-  static_assert(N == 2 || N == 4 || N == 8, "fragment count");
-  if constexpr (N == 2) {
-    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(v[0]), "+v"(v[1]));
-  } else if constexpr (N == 4) {
-    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
-  } else {
-    asm volatile("s_waitcnt lgkmcnt(0)"
-                 : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
-  }
+// A 16-byte LDS read issued the same way, for the K fragments.
+__device__ __forceinline__ u32x4_t ds_read_b128(uint32_t addr) {
+  u32x4_t v;
+  asm volatile("ds_read_b128 %0, %1" : "=v"(v) : "v"(addr));
+  return v;
+}
+
+__device__ __forceinline__ u32x2_t ds_read_b64(uint32_t addr) {
+  u32x2_t v;
+  asm volatile("ds_read_b64 %0, %1" : "=v"(v) : "v"(addr));
+  return v;
+}
+
+// LDS writes issued the same way; done (for this wavefront) at the wait of stage_barrier.
+__device__ __forceinline__ void ds_write_b64(uint32_t addr, u32x2_t v) {
+  asm volatile("ds_write_b64 %0, %1" : : "v"(addr), "v"(v) : "memory");
+}
+__device__ __forceinline__ void ds_write_b32(uint32_t addr, uint32_t v) {
+  asm volatile("ds_write_b32 %0, %1" : : "v"(addr), "v"(v) : "memory");
+}
+
+// Waits for every outstanding LDS access of the wavefront; the fragments read are tied to the wait, so no use of them
+// is scheduled before it.
+template <int N, typename V>
+__device__ __forceinline__ void tie(V (&v)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(v[i]));
+}
+template <int N, typename V>
+__device__ __forceinline__ void wait_lds_all(V (&v)[N]) {
+  asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+  tie(v);
+}
+template <int N, int M, typename V>
+__device__ __forceinline__ void wait_lds_all(V (&v)[N], V (&w)[M]) {
+  asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+  tie(v);
+  tie(w);
+}
+
+// Workgroup barrier after this wavefront's LDS accesses.  The direct-to-LDS copies it makes visible are those the
+// wavefronts have waited for (wait_vmcnt); later ones stay in flight across it.
+__device__ __forceinline__ void stage_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" : : : "memory");
+}
+
+// Two 4-value fragments as one of 8.
+__device__ __forceinline__ bf16x8_t pair(u32x2_t a, u32x2_t b) {
+  return __builtin_bit_cast(bf16x8_t, u32x4_t{a.x, a.y, b.x, b.y});
+}
+
+// A pointer that is the same in every lane, in scalar registers.
+__device__ __forceinline__ const char* scalar_ptr(const char* p) {
+  const uint64_t v = (uint64_t)p;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+  return (const char*)(((uint64_t)hi << 32) | lo);
 }
 
 __device__ __forceinline__ float wave_max_q(float v) {  // over the 4 lanes l, l^16, l^32, l^48
@@ -147,327 +247,392 @@ __device__ __forceinline__ f32x4_t bf16x4_to_f32(u32x2_t w) {
 }
 // two fp32 -> two bf16 (round to nearest even), `a` in the low half
 __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
-  return (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)a) | ((uint32_t)__builtin_bit_cast(uint16_t, (__bf16)b) << 16);
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{a, b}), bf16x2_t));
 }
 
-// Geometry of the prefix kernel for head size D.
-template <int D>
+// Geometry of the prefix kernel for head size D and RT row tiles.
+template <int D, int RT>
 struct Geo {
-  static constexpr int kRowBytes = 2 * D;                         // one cache row (bf16)
-  static constexpr int kChunks = D / 8;                           // 16-byte pieces per row
-  static constexpr int kStageBytes = kKeyBlock * kRowBytes;       // one tensor, one stage
-  static constexpr int kCopies = kStageBytes / (kWaves * 1024);   // 1 KiB copies per wavefront per tensor
+  // A stage is one 16-position key tile a wavefront.  4 wavefronts at D = 256 (two stages of 64 positions fill 128 KiB
+  // of LDS) and where 4 row tiles at D = 128 leave no room beside the rings; 8 otherwise, so that two wavefronts share
+  // a SIMD.
+  static constexpr int kWaves = D == 256 || (D == 128 && RT == 4) ? 4 : 8;
+  static constexpr int kThreads = kWaves * kWave;
+  static constexpr int kTile = 16;                          // positions of a key tile
+  static constexpr int kStage = kTile * kWaves;             // positions of a stage
+  static constexpr int kRowBytes = 2 * D;                   // one cache row (bf16)
+  static constexpr int kChunks = D / 8;                     // 16-byte pieces per row
+  static constexpr int kTileBytes = kTile * kRowBytes;      // one tensor, one tile
+  static constexpr int kCopies = kTileBytes / 1024;         // 1 KiB copies of a tile
   static constexpr int kRowsPerCopy = 1024 / kRowBytes;
-  static constexpr int kRing = 4;                                 // stages resident in LDS
-  static constexpr int kLds = kRing * 2 * kStageBytes;  // dynamic LDS (the block-table window is static)
-  static constexpr int kDTiles = D / 32;                          // 16-wide d tiles per wavefront (half of D)
-  static constexpr int kDChunks = D / 32;                         // 32-d MFMA steps of a score
-  static_assert(kCopies >= 1 && kStageBytes % (kWaves * 1024) == 0, "stage must split into wave copies");
-  static_assert(kDTiles >= 1, "head size too small");
-  static_assert(kLds + kTablePages * 4 <= kMaxDynLds + 8 * 1024 - 256, "LDS budget");
-  static_assert(2 * 4 * kDTiles * 64 * 16 + 2 * 4 * 64 * 8 <= kLds, "key-tile merge fits the ring");
+  static constexpr int kDChunks = D / 32;                   // 32-d MFMA steps of a score
+  // The output's 16-wide d tiles over the wavefronts: kOwn for each of kDGroups; wavefronts beyond those (D = 64) take
+  // every other row tile.
+  static constexpr int kDTiles = D / 16;
+  static constexpr int kDGroups = kDTiles < kWaves ? kDTiles : kWaves;
+  static constexpr int kOwn = kDTiles / kDGroups;
+  static constexpr int kRowGroups = kWaves / kDGroups;
+  static constexpr int kOwnRows = (RT + kRowGroups - 1) / kRowGroups;
+  // LDS: K and V tiles [2][wavefront], then the softmax weights [2][wavefront][RT][64 lanes x 8 bytes].
+  static constexpr int kWeights = 2 * kWaves * 2 * kTileBytes;
+  static constexpr int kLds = kWeights + 2 * kWaves * RT * 512;
+  static_assert(kLds + RT * kWaves * 128 + 256 <= (int)kMaxLds, "LDS budget");
   // The 16-byte piece of row n that lands at LDS position p is piece p ^ swz(n): 16 consecutive rows
   // read at one piece index then hit 16 distinct bank groups.
   __device__ static __forceinline__ int swz(int n) { return kChunks >= 16 ? (n & 15) : ((n >> 1) & 7); }
 };
 
-// One wavefront per SIMD (128 KiB of LDS per workgroup at D = 256): the whole register file is usable.
-template <int D, int RT>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void spec_prefix_kernel(
-    AttnArgs a) {
-  using Gm = Geo<D>;
-  constexpr int kRing = Gm::kRing;
-  constexpr int NJ = Gm::kCopies;
+// ALIGNED: the page size is a multiple of 16, so a key tile lies in one page (splits start on multiples of 32) and a copy
+// takes one scalar base.  Otherwise each lane finds its row's page among the two a tile can touch.  Both forms are free
+// of branches, so that the compiler can count the vector-memory instructions outstanding.
+template <int D, int RT, bool ALIGNED>
+__global__ __launch_bounds__((Geo<D, RT>::kThreads))
+__attribute__((amdgpu_waves_per_eu((Geo<D, RT>::kWaves / 4), (Geo<D, RT>::kWaves / 4)))) void
+spec_prefix_kernel(AttnArgs a) {
+  using Gm = Geo<D, RT>;
+  constexpr int kWaves = Gm::kWaves;
+  constexpr int NK = Gm::kCopies;
   extern __shared__ __align__(16) uint8_t lds[];
-  __shared__ int32_t tbl[kTablePages];  // block-table entries of the current window
-
-  const int split = blockIdx.x;
-  const int b = blockIdx.y / a.HKV;
-  const int hkv = blockIdx.y - b * a.HKV;
-  const int seq = a.seq_lens[b];
-  const int prefix = seq - a.Q > 0 ? seq - a.Q : 0;
-  const int chunk = split_chunk(prefix, a.splits, a.min_chunk);
-  const int n_active = prefix > 0 ? (prefix + chunk - 1) / chunk : 0;
-  // Split s takes positions [s * chunk, min((s + 1) * chunk, prefix)); the last active split (split 0
-  // when the prefix is empty) also takes this step's in-flight positions [prefix, seq).  Query qi sees
-  // the positions up to seq - q_len + qi, which include the whole prefix, so one causal bound per
-  // row covers both kinds of position.
-  const int last_split = n_active > 0 ? n_active - 1 : 0;
-  const int start = split * chunk;
-  const int end = split == last_split ? seq : min(start + chunk, prefix);
-  if (split > last_split || start >= end) {
-    // no position here: the split's rows get log-sum-exp -inf, so the combine kernel can read every
-    // split without knowing the sequence length (uniform: the whole workgroup leaves)
-    const int64_t part = ((int64_t)blockIdx.y * a.splits + split) * a.R;
-    for (int r = threadIdx.x; r < a.R; r += kThreads) a.lse_part[part + r] = -__builtin_inff();
-    return;
-  }
+  __shared__ float row_exchange[RT][kWaves][16];      // a value a row and wavefront: the maxima, at the end the sums
+  __shared__ __align__(16) uint32_t moved[2][8];      // a wavefront found a score above the reference, stage parity
 
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int hkv = blockIdx.y;
+  int b = blockIdx.z, split = blockIdx.x, seq, chunk, n = 0, first = 0;
+  if (a.plan != nullptr) {
+    int total;
+    balance(a, lane, seq, chunk, n, first, total);
+    if ((int)blockIdx.x >= total) return;  // a slot of no request: the combine kernel reads the used ones only
+    b = 63 - __builtin_clzll(__ballot(lane < a.B && first <= (int)blockIdx.x));
+    split = blockIdx.x - __builtin_amdgcn_readlane(first, b);
+    seq = __builtin_amdgcn_readlane(seq, b);
+    chunk = __builtin_amdgcn_readfirstlane(chunk);
+  }
+
+  // Packed query rows: B fragments of the score product (rows >= R repeat row R - 1), requested first, so that they
+  // arrive while the sequence length and the block ids do.
   const int l16 = lane & 15;
   const int qg = lane >> 4;
-  const int kh = wave & 1;   // key tile of each stage
-  const int dh = wave >> 1;  // half of the head dimension
-
-  // ---- packed query rows: B fragments of the score product (rows >= R repeat row R - 1) ----
   bf16x8_t qf[RT][Gm::kDChunks];
-  int last[RT];  // last visible position of the lane's score row in each row tile
+  int q_index[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
     const int r = min(rt * 16 + l16, a.R - 1);
-    const int qi = r / a.G;
-    const int h = hkv * a.G + (r - qi * a.G);
-    last[rt] = seq - a.Q + qi;
-    const uint16_t* qrow = a.q + (int64_t)(b * a.Q + qi) * a.sq_t + (int64_t)h * a.sq_h + qg * 8;
+    q_index[rt] = divide(r, a.by_g);
+    const int h = hkv * a.G + (r - q_index[rt] * a.G);
+    const uint16_t* qrow = a.q + (int64_t)(b * a.Q + q_index[rt]) * a.sq_t + (int64_t)h * a.sq_h + qg * 8;
 #pragma unroll
     for (int c = 0; c < Gm::kDChunks; ++c) qf[rt][c] = *reinterpret_cast<const bf16x8_t*>(qrow + c * 32);
   }
 
-  // ---- copy schedule: per stage, wavefront `wave` moves NJ KiB of K and NJ KiB of V.  Lane offsets
-  // within a stage are fixed; per stage only the page bases change (computed in scalar registers) ----
+  if (a.plan == nullptr) seq = a.seq_lens[b];
+  const int prefix = seq - a.Q > 0 ? seq - a.Q : 0;
+  if (a.plan == nullptr) chunk = split_chunk(prefix, a);
+  const int64_t part = (((int64_t)b * (a.plan != nullptr ? 0 : a.HKV) + hkv) * a.splits + blockIdx.x) * a.R;
+  // Split s takes positions [s * chunk, min((s + 1) * chunk, prefix)); the last active split (split 0
+  // when the prefix is empty) also takes this step's in-flight positions [prefix, seq).  Query qi sees
+  // the positions up to seq - q_len + qi, which include the whole prefix, so one causal bound per
+  // row covers both kinds of position.
+  const int start = split * chunk;
+  const bool active = split == 0 || start < prefix;
+  const int end = start + chunk >= prefix ? seq : start + chunk;
+  if (a.plan != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && wave == 0 && lane < a.B) a.plan[lane] = make_int2(first, n);
+  if (!active || start >= end) {
+    // no position here: the split's rows get log-sum-exp -inf, so the combine kernel can read every
+    // split without knowing the sequence length (uniform: the whole workgroup leaves)
+    for (int r = threadIdx.x; r < a.R; r += Gm::kThreads) a.lse_part[part + r] = -__builtin_inff();
+    return;
+  }
+  int last[RT];  // last visible position of the lane's score row in each row tile
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) last[rt] = seq - a.Q + q_index[rt];
+
+  // ---- this wavefront's key tiles: tile `wave` of every stage (past the end: the split's last tile again) ----
+  const int n_tiles = (end - start + Gm::kTile - 1) / Gm::kTile;
+  const int n_stages = (n_tiles + kWaves - 1) / kWaves;
   const int32_t* bt_row = a.bt + (int64_t)b * a.sbt;
   const char* kbytes = reinterpret_cast<const char*>(a.kc + (int64_t)hkv * a.sk_h);
   const char* vbytes = reinterpret_cast<const char*>(a.vc + (int64_t)hkv * a.sv_h);
-  int row_of[NJ];
-  uint32_t koff[NJ], voff[NJ], poff[NJ];  // byte offsets: row t's piece, and the piece in row 0
-#pragma unroll
-  for (int j = 0; j < NJ; ++j) {
-    const int t = (wave * NJ + j) * Gm::kRowsPerCopy + lane / Gm::kChunks;
-    const int piece = (lane % Gm::kChunks) ^ Gm::swz(t);
-    row_of[j] = t;
-    poff[j] = piece * 16;
-    koff[j] = (uint32_t)(t * a.sk_t * 2) + poff[j];
-    voff[j] = (uint32_t)(t * a.sv_t * 2) + poff[j];
-  }
+  const int last_page = divide(end - 1, a.by_page);
 
-  // byte offsets (within a stage's V rows) of this lane's transposing reads, one per d tile
-  uint32_t vt_off[Gm::kDTiles];
-  {
-    const int n = kh * 16 + 4 * (lane >> 4) + ((lane >> 2) & 3);
-    const int q4 = lane & 3;
+  // Block ids of 64 of the wavefront's tiles, one a lane: the page of the tile's first row (and the page after it: a
+  // tile of 16 rows touches at most two pages of 16 or more), and the first row's place in its page.
+  int blk0, blk1 = 0, in_page;
+  auto load_blocks = [&](int base) {
+    const int pos = start + min(wave + (base + lane) * kWaves, n_tiles - 1) * Gm::kTile;
+    const int pg = divide(pos, a.by_page);
+    in_page = pos - pg * a.page;
+    blk0 = bt_row[pg];
+    if constexpr (!ALIGNED) blk1 = bt_row[min(pg + 1, last_page)];
+  };
+  load_blocks(0);
+  wait_vmcnt<0>();  // the queries too: none may be outstanding when the copies are counted below
+
+  // ---- copies: lane l of copy j moves the 16-byte piece p of row n = j * kRowsPerCopy + l / kChunks of the tile to
+  // piece l % kChunks = p ^ swz(n) ----
+  const int t_lane = lane / Gm::kChunks;
+  auto piece = [&](int j) {
+    return (uint32_t)(((lane % Gm::kChunks) ^ Gm::swz(j * Gm::kRowsPerCopy + t_lane)) * 16);
+  };
+  struct Where {
+    int blk0, blk1, in_page;
+  };
+  auto where = [&](int stage) {
+    const int i = stage & (kWave - 1);
+    return Where{__builtin_amdgcn_readlane(blk0, i), ALIGNED ? 0 : __builtin_amdgcn_readlane(blk1, i),
+                 __builtin_amdgcn_readlane(in_page, i)};
+  };
+  auto copy = [&](const char* bytes, int64_t sb, int64_t st, Where at, int stage, uint8_t* dst) {
+    const char* base = bytes + (at.blk0 * sb + at.in_page * st) * 2;
 #pragma unroll
-    for (int dt = 0; dt < Gm::kDTiles; ++dt) {
-      const int d = (dh * Gm::kDTiles + dt) * 16 + 4 * q4;
-      vt_off[dt] = (uint32_t)(n * Gm::kRowBytes + (((d >> 3) ^ Gm::swz(n)) << 4) + (d & 7) * 2);
+    for (int j = 0; j < NK; ++j) {
+      const char* p;
+      if constexpr (ALIGNED) {  // a scalar base and a 32-bit lane offset; rows past the end are the page's own
+        p = scalar_ptr(base + (int64_t)j * Gm::kRowsPerCopy * 2 * st) + ((uint32_t)(t_lane * (int)st * 2) + piece(j));
+      } else {  // rows past the end re-read the tile's first row; rows past the page count back from the next one
+        const char* base1 = bytes + (at.blk1 * sb + (at.in_page - a.page) * st) * 2;
+        const int pos = start + min(wave + stage * kWaves, n_tiles - 1) * Gm::kTile;
+        int row = j * Gm::kRowsPerCopy + t_lane;
+        row = row < end - pos ? row : 0;
+        p = (row < a.page - at.in_page ? base : base1) + row * st * 2 + piece(j);
+      }
+      __builtin_amdgcn_global_load_lds((gptr_t)p, (lptr_t)(dst + j * 1024), 16, 0, kNonTemporal);
     }
-  }
+  };
+  // slot (stage & 1) of a tensor: [2][kWaves] tiles of K, then of V
+  auto k_slot = [&](int stage, int w) { return lds + ((stage & 1) * kWaves + w) * Gm::kTileBytes; };
+  auto v_slot = [&](int stage, int w) { return lds + ((2 + (stage & 1)) * kWaves + w) * Gm::kTileBytes; };
+  auto copy_k = [&](Where at, int stage) { copy(kbytes, a.sk_b, a.sk_t, at, stage, k_slot(stage, wave)); };
+  auto copy_v = [&](Where at, int stage) { copy(vbytes, a.sv_b, a.sv_t, at, stage, v_slot(stage, wave)); };
 
-  // online softmax state: m_ref is the row's exponent reference, moved only when a score exceeds it
-  // by more than kRescale (log2 units), so the probabilities stay below 2^kRescale and the
-  // accumulators are rarely rescaled; the result equals the running-maximum form up to rounding
+  if (wave < n_tiles) {  // a split of less than a stage: the other wavefronts have no tile (and no later copy to count)
+    copy_k(where(0), 0);
+    copy_v(where(0), 0);
+  }
+  Where next = where(1);  // the next stage's tile (its V is requested a stage after its K)
+  if (n_stages > 1) copy_k(next, 1);
+
+  // byte offsets of this lane's LDS reads in a tile: the K fragment of d step c at k_off ^ 64 c, the transposing V
+  // read of d tile dt at v_off ^ 32 dt (the swizzle's bits and the step's do not overlap)
+  const uint32_t k_off = (uint32_t)(l16 * Gm::kRowBytes + ((qg ^ Gm::swz(l16)) << 4));
+  uint32_t v_off;
+  {
+    const int n = 4 * (lane >> 4) + ((lane >> 2) & 3);
+    const int d = 4 * (lane & 3);
+    v_off = (uint32_t)(n * Gm::kRowBytes + (((d >> 3) ^ Gm::swz(n)) << 4) + (d & 7) * 2);
+  }
+  // the output tiles of this wavefront: d tiles dg * kOwn .. + kOwn - 1 of the row tiles rg, rg + kRowGroups, ...
+  const int dg = wave % Gm::kDGroups;
+  const int rg = wave / Gm::kDGroups;
+  v_off ^= 32 * (dg * Gm::kOwn);
+
+  // Online softmax state.  m_ref is the row's exponent reference, the same in every wavefront, moved only when a
+  // score exceeds it by more than kRescale (log2 units), so the weights stay below 2^kRescale and the accumulators are
+  // rarely rescaled; the result equals the running-maximum form up to rounding.  l_run sums this wavefront's weights
+  // (its key tiles, its lanes' positions).
   constexpr float kRescale = 8.f;
   float m_ref[RT], l_run[RT];
-  f32x4_t o_acc[RT][Gm::kDTiles];
+  f32x4_t o_acc[Gm::kOwnRows][Gm::kOwn];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
     m_ref[rt] = -__builtin_inff();
     l_run[rt] = 0.f;
-#pragma unroll
-    for (int dt = 0; dt < Gm::kDTiles; ++dt) o_acc[rt][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
-
-  // The split is walked in windows of at most kTablePages pages (one window unless the split spans
-  // more pages than that); each window's block-table entries are read into LDS first, so inside the
-  // pipelined loop the only vector-memory instructions are the stage copies and the explicit vmcnt
-  // waits below count exactly those.
-  for (int wstart = start; wstart < end;) {
-    const int p0 = wstart / a.page;
-    const int wend = min(end, (p0 + kTablePages) * a.page);
-    const int npg = (wend - 1) / a.page - p0 + 1;
-    for (int i = threadIdx.x; i < npg; i += kThreads) tbl[i] = bt_row[p0 + i];
-    wait_vmcnt<0>();  // the query loads too: nothing may be left in flight before the exact waits below
-    __syncthreads();
-    const int nst = (wend - wstart + kKeyBlock - 1) / kKeyBlock;
-
-    // Stages are copied in order; the next one starts in page pg_n at in-page offset og_n.  A stage
-    // of 32 positions spans at most 3 pages of >= 16 positions.
-    int issued = 0, pg_n = p0, og_n = wstart - p0 * a.page;
-    auto copy_next = [&]() {
-      const int st = issued++;
-      uint8_t* slot = lds + (st % kRing) * 2 * Gm::kStageBytes;
-      const int nvalid = min(kKeyBlock, wend - (wstart + st * kKeyBlock));
-      const int bnd1 = a.page - og_n;  // rows >= bnd1 lie in the next page, rows >= bnd2 in the one after
-      const int bnd2 = bnd1 + a.page;
-      const int e0 = pg_n - p0;
-      const int64_t blk0 = __builtin_amdgcn_readfirstlane(tbl[e0]);
-      const int64_t kb0 = (blk0 * a.sk_b + (int64_t)og_n * a.sk_t) * 2;
-      const int64_t vb0 = (blk0 * a.sv_b + (int64_t)og_n * a.sv_t) * 2;
-      if (bnd1 >= kKeyBlock && nvalid == kKeyBlock) {
-        // the whole stage lies in one page (uniform): one base per tensor
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          const int copy = wave * NJ + j;
-          __builtin_amdgcn_global_load_lds((gptr_t)(kbytes + kb0 + koff[j]), (lptr_t)(slot + copy * 1024), 16, 0, 0);
-          __builtin_amdgcn_global_load_lds((gptr_t)(vbytes + vb0 + voff[j]),
-                                           (lptr_t)(slot + Gm::kStageBytes + copy * 1024), 16, 0, 0);
-        }
+  for (int q = 0; q < Gm::kOwnRows; ++q)
+#pragma unroll
+    for (int u = 0; u < Gm::kOwn; ++u) o_acc[q][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+#pragma unroll 1
+  for (int st = 0; st < n_stages; ++st) {
+    // The copies are requested in the order K0 V0 K1 | K2 V1 | K3 V2 | ...  K of stage 0 has landed once V0 and K1
+    // alone are outstanding, K of stage 1 with K2 and V1; a later stage's did before the last barrier (it is ahead of
+    // that stage's V, which every wavefront waited for).
+    if (st < 2) {
+      if (n_stages > 1 + st) {
+        wait_vmcnt<2 * NK>();
       } else {
-        const int64_t blk1 = __builtin_amdgcn_readfirstlane(tbl[min(e0 + 1, npg - 1)]);
-        const int64_t blk2 = __builtin_amdgcn_readfirstlane(tbl[min(e0 + 2, npg - 1)]);
-        const int64_t kb1 = (blk1 * a.sk_b + (int64_t)(og_n - a.page) * a.sk_t) * 2;
-        const int64_t kb2 = (blk2 * a.sk_b + (int64_t)(og_n - 2 * a.page) * a.sk_t) * 2;
-        const int64_t vb1 = (blk1 * a.sv_b + (int64_t)(og_n - a.page) * a.sv_t) * 2;
-        const int64_t vb2 = (blk2 * a.sv_b + (int64_t)(og_n - 2 * a.page) * a.sv_t) * 2;
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          const bool valid = row_of[j] < nvalid;  // rows past the window re-read the stage's first row
-          const int t = valid ? row_of[j] : 0;
-          const int64_t kb = t >= bnd2 ? kb2 : (t >= bnd1 ? kb1 : kb0);
-          const int64_t vb = t >= bnd2 ? vb2 : (t >= bnd1 ? vb1 : vb0);
-          const int copy = wave * NJ + j;
-          __builtin_amdgcn_global_load_lds((gptr_t)(kbytes + kb + (valid ? koff[j] : poff[j])),
-                                           (lptr_t)(slot + copy * 1024), 16, 0, 0);
-          __builtin_amdgcn_global_load_lds((gptr_t)(vbytes + vb + (valid ? voff[j] : poff[j])),
-                                           (lptr_t)(slot + Gm::kStageBytes + copy * 1024), 16, 0, 0);
-        }
+        wait_vmcnt<NK>();
       }
-      og_n += kKeyBlock;
-      while (og_n >= a.page) {
-        og_n -= a.page;
-        ++pg_n;
+    }
+
+    Where after_next;
+
+    // S^T of the wavefront's key tile: positions 4 qg + i, row 16 rt + l16
+    f32x4_t sc[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) sc[rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    {
+      const uint32_t ks = lds_addr(k_slot(st, wave));
+      u32x4_t kf[Gm::kDChunks];
+#pragma unroll
+      for (int c = 0; c < Gm::kDChunks; ++c) kf[c] = ds_read_b128(ks + (k_off ^ (64 * c)));
+      wait_lds_all<Gm::kDChunks>(kf);
+      after_next = next;
+      if (st + 2 < n_stages) {  // the K reads have returned: their slot is free
+        if (((st + 2) & (kWave - 1)) == 0) {
+          load_blocks(st + 2);
+          wait_vmcnt<0>();  // here, once in 64 stages, and not at every use of the block ids
+        }
+        after_next = where(st + 2);
+        copy_k(after_next, st + 2);
+      }
+#pragma unroll
+      for (int c = 0; c < Gm::kDChunks; ++c)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+          sc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[c]), qf[rt][c], sc[rt], 0, 0, 0);
+    }
+
+    // scores in base 2; a tile wholly inside every row's visible range needs no mask
+    const int pos = start + (wave + st * kWaves) * Gm::kTile;
+    const int pos0 = pos + qg * 4;
+    float mx[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) sc[rt] *= a.qk_scale;
+    if (pos + Gm::kTile > end || pos + Gm::kTile - 1 > seq - a.Q) {
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sc[rt][i] = pos0 + i < end && pos0 + i <= last[rt] ? sc[rt][i] : -__builtin_inff();
+    }
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) mx[rt] = fmaxf(fmaxf(sc[rt][0], sc[rt][1]), fmaxf(sc[rt][2], sc[rt][3]));
+
+    // The weights against the present references, rounded to bf16, to the other wavefronts through LDS: lane (qg, l16)
+    // holds those of 4 positions of one row, its part of the B fragment of O^T = V^T P^T.
+    float sum[RT];
+    const uint32_t w_slot = lds_addr(lds) + Gm::kWeights + (uint32_t)((st & 1) * kWaves * RT * 512) + lane * 8;
+    auto weigh = [&]() {
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+        const float m_base = m_ref[rt] == -__builtin_inff() ? 0.f : m_ref[rt];  // -inf: a row that has seen nothing yet
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = fast_exp2(sc[rt][i] - m_base);
+        sum[rt] = (v[0] + v[1]) + (v[2] + v[3]);
+        ds_write_b64(w_slot + (wave * RT + rt) * 512, u32x2_t{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])});
       }
     };
-
-    // prologue: stages 0 .. kRing-2 in flight
+    bool move = st == 0;
+    if (!move) {
+      bool above = false;
 #pragma unroll
-    for (int s = 0; s < kRing - 1; ++s)
-      if (s < nst) copy_next();
-
-    constexpr int kCopiesPerStage = 2 * NJ;  // vector-memory instructions of one stage
-    for (int st = 0; st < nst; ++st) {
-      // Stage st has landed once at most the later issued stages' copies are outstanding.  Stages
-      // up to st + kRing - 2 have been issued; st + kRing - 1 goes out after the barrier below.
-      const int after = min(kRing - 2, nst - 1 - st);
-      if (after >= 2) {
-        wait_vmcnt<2 * kCopiesPerStage>();
-      } else if (after == 1) {
-        wait_vmcnt<kCopiesPerStage>();
+      for (int rt = 0; rt < RT; ++rt) above |= mx[rt] > m_ref[rt] + kRescale;
+      weigh();
+      ds_write_b32(lds_addr(&moved[st & 1][wave]), __any(above) ? 1u : 0u);  // every lane the same word
+    }
+    // V of this stage has landed once only the K copies requested after it are outstanding
+    if (st + 2 >= n_stages) {
+      if (st == 0 && n_stages > 1) {
+        wait_vmcnt<NK>();
       } else {
         wait_vmcnt<0>();
       }
-      ring_barrier();
-      // Refill the slot every wavefront finished with before this barrier (stage st - 1's); three
-      // stages are then in flight while this one is computed.
-      if (st + kRing - 1 < nst) copy_next();
-      __builtin_amdgcn_sched_barrier(0);
-
-      const uint8_t* ks = lds + (st % kRing) * 2 * Gm::kStageBytes;
-      const uint8_t* vs = ks + Gm::kStageBytes;
-      const int sbase = wstart + st * kKeyBlock;
-
-      // S^T tile of this wavefront's key tile kh: positions 16 kh + 4 qg + i, row 16 rt + l16
-      f32x4_t sc[RT];
+    } else if (st == 0) {
+      wait_vmcnt<2 * NK>();
+    } else {
+      wait_vmcnt<NK>();
+    }
+    if (!move) {
+      stage_barrier();
+      u32x4_t f[kWaves / 4];
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt) sc[rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      const int n_k = kh * 16 + l16;
+      for (int i = 0; i < kWaves / 4; ++i) f[i] = ds_read_b128(lds_addr(&moved[st & 1][4 * i]));
+      wait_lds_all<kWaves / 4>(f);
+      uint32_t any = 0;
 #pragma unroll
-      for (int c = 0; c < Gm::kDChunks; ++c) {
-        const bf16x8_t kf = *reinterpret_cast<const bf16x8_t*>(
-            ks + n_k * Gm::kRowBytes + (((4 * c + qg) ^ Gm::swz(n_k)) << 4));
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-          sc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[rt][c], sc[rt], 0, 0, 0);
-      }
-
-      // softmax weights in base 2; the lane's 4 probabilities are its B fragment of O^T = V^T P^T.
-      // A stage wholly inside every row's visible range needs no mask.
-      const int pos0 = sbase + kh * 16 + qg * 4;
-      const bool full = sbase + kKeyBlock <= wend && sbase + kKeyBlock - 1 <= seq - a.Q;
-      s16x4_t pf[RT];
+      for (int i = 0; i < kWaves / 4; ++i) any |= (f[i].x | f[i].y) | (f[i].z | f[i].w);
+      move = __builtin_amdgcn_readfirstlane(any) != 0;
+    }
+    if (move) {  // the same in every wavefront: the rows' new references, and the weights again
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
-        float v[4];
-        if (full) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) v[i] = sc[rt][i] * a.qk_scale;
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            v[i] = pos0 + i < wend && pos0 + i <= last[rt] ? sc[rt][i] * a.qk_scale : -__builtin_inff();
-        }
-        const float mx = fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3]));
-        if (__any(mx > m_ref[rt] + kRescale)) {  // wave-uniform: move the references of all rows
-          const float m_new = fmaxf(m_ref[rt], wave_max_q(mx));
-          // -inf only for a row that has seen no position yet: exponent base 0 then
-          const float alpha = fast_exp2(m_ref[rt] - (m_new == -__builtin_inff() ? 0.f : m_new));
-          l_run[rt] *= alpha;
-#pragma unroll
-          for (int dt = 0; dt < Gm::kDTiles; ++dt) o_acc[rt][dt] *= alpha;
-          m_ref[rt] = m_new;
-        }
-        const float m_base = m_ref[rt] == -__builtin_inff() ? 0.f : m_ref[rt];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = fast_exp2(v[i] - m_base);
-        l_run[rt] += (v[0] + v[1]) + (v[2] + v[3]);
-        pf[rt] = __builtin_bit_cast(s16x4_t, u32x2_t{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])});
+        mx[rt] = wave_max_q(mx[rt]);
+        ds_write_b32(lds_addr(&row_exchange[rt][wave][l16]), __float_as_uint(mx[rt]));  // four lanes the same word
       }
+      stage_barrier();
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+        float m_new = m_ref[rt];
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) m_new = fmaxf(m_new, row_exchange[rt][w][l16]);
+        const float alpha = fast_exp2(m_ref[rt] - (m_new == -__builtin_inff() ? 0.f : m_new));
+        m_ref[rt] = m_new;
+        l_run[rt] *= alpha;
+        if (st > 0 && rt % Gm::kRowGroups == rg) {
+#pragma unroll
+          for (int u = 0; u < Gm::kOwn; ++u) o_acc[rt / Gm::kRowGroups][u] *= alpha;
+        }
+      }
+      weigh();
+      stage_barrier();
+    }
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) l_run[rt] += sum[rt];
+    // every wavefront is past the previous stage's V
+    if (st + 1 < n_stages) copy_v(next, st + 1);
+    next = after_next;
 
-      // O^T += V^T P^T over this wavefront's d half and key tile (k slot 4 qg + i = position 4 qg + i).
-      // The V^T fragment of a d tile comes from one transposing LDS read: lane 16 g + 4 j + q points at
-      // the 8 bytes of row 4 g + j holding d values d0 + 4 q .. d0 + 4 q + 3, and the read hands lane
-      // 16 g + i the values V[4 g + j][d0 + i], j = 0..3.
-      u32x2_t vf[Gm::kDTiles];
-      const uint32_t vs_lds = lds_addr(vs);
+    // O^T += V^T P^T over the stage, two key tiles an instruction: k slot (qg, j) is position 4 qg + j of the first
+    // tile for j < 4 and 4 qg + j - 4 of the second for j >= 4.  The V^T fragment of a d tile comes from one
+    // transposing LDS read a key tile: lane 16 g + 4 j + q points at the 8 bytes of row 4 g + j holding d values
+    // d0 + 4 q .. d0 + 4 q + 3, and the read hands lane 16 g + i the values V[4 g + j][d0 + i], j = 0..3.
+    u32x2_t vf[Gm::kOwn * kWaves], pf[Gm::kOwnRows * kWaves];
 #pragma unroll
-      for (int dt = 0; dt < Gm::kDTiles; ++dt) vf[dt] = ds_read_tr16_b64(vs_lds + vt_off[dt]);
-      wait_lds_all<Gm::kDTiles>(vf);
+    for (int w = 0; w < kWaves; ++w) {
+      const uint32_t vs = lds_addr(v_slot(st, w));
 #pragma unroll
-      for (int dt = 0; dt < Gm::kDTiles; ++dt) {
-        const s16x4_t a_frag = __builtin_bit_cast(s16x4_t, vf[dt]);
+      for (int u = 0; u < Gm::kOwn; ++u) vf[w * Gm::kOwn + u] = ds_read_tr16_b64(vs + (v_off ^ (32 * u)));
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-          o_acc[rt][dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a_frag, pf[rt], o_acc[rt][dt], 0, 0, 0);
+      for (int q = 0; q < Gm::kOwnRows; ++q)
+        pf[w * Gm::kOwnRows + q] = ds_read_b64(w_slot + (w * RT + min(q * Gm::kRowGroups + rg, RT - 1)) * 512);
+    }
+    wait_lds_all(vf, pf);
+    if (st + 1 == n_stages && start + n_stages * Gm::kStage > end) {
+      // Rows past the end hold whatever the page, or the slot, does (perhaps NaN): their weight is 0, their V made 0.
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) {
+        const int p0 = start + (w + st * kWaves) * Gm::kTile + qg * 4;
+        const uint32_t w0 = (p0 < end ? 0xffffu : 0u) | (p0 + 1 < end ? 0xffff0000u : 0u);
+        const uint32_t w1 = (p0 + 2 < end ? 0xffffu : 0u) | (p0 + 3 < end ? 0xffff0000u : 0u);
+#pragma unroll
+        for (int u = 0; u < Gm::kOwn; ++u) vf[w * Gm::kOwn + u] &= u32x2_t{w0, w1};
       }
     }
-    wait_vmcnt<0>();
-    __syncthreads();  // the next window rewrites the table and the ring
-    wstart = wend;
+#pragma unroll
+    for (int w = 0; w < kWaves; w += 2)
+#pragma unroll
+      for (int u = 0; u < Gm::kOwn; ++u)
+#pragma unroll
+        for (int q = 0; q < Gm::kOwnRows; ++q)
+          o_acc[q][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              pair(vf[w * Gm::kOwn + u], vf[(w + 1) * Gm::kOwn + u]),
+              pair(pf[w * Gm::kOwnRows + q], pf[(w + 1) * Gm::kOwnRows + q]), o_acc[q][u], 0, 0, 0);
   }
 
-  // ---- merge the two key tiles' states (wavefront kh = 1 hands its state to kh = 0 of the same d
-  // half through the now idle ring), then the partial output (normalised) and base-2 log-sum-exp of
-  // each packed row; a row that saw no position (possible only in the split holding the in-flight
-  // positions) is written as 0 with log-sum-exp -inf ----
-  float* xo = reinterpret_cast<float*>(lds);                        // [2][RT][kDTiles][64] x f32x4
-  float* xs = xo + 2 * RT * Gm::kDTiles * kWave * 4;               // [2][RT][64] x (m, l)
-  float l_tot[RT];
+  // ---- the rows' sums over the wavefronts, then the partial output (normalised) and base-2 log-sum-exp of each packed
+  // row; a row that saw no position (possible only in the split holding the in-flight positions) is written as 0 with
+  // log-sum-exp -inf ----
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) l_tot[rt] = wave_sum_q(l_run[rt]);
-  if (kh == 1) {
+  for (int rt = 0; rt < RT; ++rt) l_run[rt] = wave_sum_q(l_run[rt]);
+  stage_barrier();  // the last maxima have been read
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-#pragma unroll
-      for (int dt = 0; dt < Gm::kDTiles; ++dt)
-        *reinterpret_cast<f32x4_t*>(xo + (((dh * RT + rt) * Gm::kDTiles + dt) * kWave + lane) * 4) = o_acc[rt][dt];
-      xs[((dh * RT + rt) * kWave + lane) * 2] = m_ref[rt];
-      xs[((dh * RT + rt) * kWave + lane) * 2 + 1] = l_tot[rt];
-    }
-  }
-  __syncthreads();
-  if (kh == 1) return;
-  const int64_t part = ((int64_t)blockIdx.y * a.splits + split) * a.R;
+  for (int rt = 0; rt < RT; ++rt) ds_write_b32(lds_addr(&row_exchange[rt][wave][l16]), __float_as_uint(l_run[rt]));
+  stage_barrier();
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
-    const float m1 = xs[((dh * RT + rt) * kWave + lane) * 2];
-    const float l1 = xs[((dh * RT + rt) * kWave + lane) * 2 + 1];
-    const float mt = fmaxf(m_ref[rt], m1);
-    const float mb = mt == -__builtin_inff() ? 0.f : mt;
-    const float a0 = fast_exp2(m_ref[rt] - mb), a1 = fast_exp2(m1 - mb);
-    const float lt = l_tot[rt] * a0 + l1 * a1;
-    const float inv = lt > 0.f ? 1.f / lt : 0.f;
     const int r = rt * 16 + l16;
-    if (r < a.R) {
-      float* orow = a.o_part + (part + r) * D;
+    if (rt % Gm::kRowGroups != rg || r >= a.R) continue;
+    float lt = 0.f;
 #pragma unroll
-      for (int dt = 0; dt < Gm::kDTiles; ++dt) {
-        const f32x4_t o1 =
-            *reinterpret_cast<const f32x4_t*>(xo + (((dh * RT + rt) * Gm::kDTiles + dt) * kWave + lane) * 4);
-        *reinterpret_cast<f32x4_t*>(orow + (dh * Gm::kDTiles + dt) * 16 + qg * 4) =
-            (o_acc[rt][dt] * a0 + o1 * a1) * inv;
-      }
-      if (dh == 0 && qg == 0) a.lse_part[part + r] = lt > 0.f ? mt + __log2f(lt) : -__builtin_inff();
-    }
+    for (int w = 0; w < kWaves; ++w) lt += row_exchange[rt][w][l16];
+    const float inv = lt > 0.f ? 1.f / lt : 0.f;
+    float* orow = a.o_part + (part + r) * D + dg * Gm::kOwn * 16 + qg * 4;
+#pragma unroll
+    for (int u = 0; u < Gm::kOwn; ++u) *reinterpret_cast<f32x4_t*>(orow + u * 16) = o_acc[rt / Gm::kRowGroups][u] * inv;
+    if (dg == 0 && qg == 0) a.lse_part[part + r] = lt > 0.f ? m_ref[rt] + __log2f(lt) : -__builtin_inff();
   }
 }
 
@@ -490,7 +655,7 @@ __global__ __launch_bounds__(kThreads) void spec_combine_kernel(AttnArgs a) {
   const int d0 = blockIdx.y * kCombSlice;
   const int tok = row / a.H;
   const int h = row - tok * a.H;
-  const int b = tok / a.Q;
+  const int b = __builtin_amdgcn_readfirstlane(tok / a.Q);
   const int qi = tok - b * a.Q;
   const int hkv = h / a.G;
   const int r = qi * a.G + (h - hkv * a.G);
@@ -499,16 +664,22 @@ __global__ __launch_bounds__(kThreads) void spec_combine_kernel(AttnArgs a) {
 
   float m = -__builtin_inff(), l = 0.f;
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-  const int64_t part0 = ((int64_t)(b * a.HKV + hkv) * a.splits) * a.R + r;
+  int parts = a.splits;
+  int64_t part0 = ((int64_t)(b * a.HKV + hkv) * a.splits) * a.R + r;
+  if (a.plan != nullptr) {
+    const int2 place = a.plan[b];
+    parts = place.y;
+    part0 = ((int64_t)hkv * a.splits + place.x) * a.R + r;
+  }
   // group grp merges the parts grp, grp + NGRP, ...
-  for (int base = grp; base < a.splits; base += NGRP * kBatch) {
+  for (int base = grp; base < parts; base += NGRP * kBatch) {
     float e[kBatch];
     f32x4_t o[kBatch];
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
       const int i = base + u * NGRP;
       e[u] = -__builtin_inff();
-      if (i < a.splits) {
+      if (i < parts) {
         const int64_t idx = part0 + (int64_t)i * a.R;
         e[u] = a.lse_part[idx];
         o[u] = *reinterpret_cast<const f32x4_t*>(a.o_part + idx * D + d0 + dq * 4);
@@ -553,21 +724,34 @@ __global__ __launch_bounds__(kThreads) void spec_combine_kernel(AttnArgs a) {
 
 typedef void (*KernelFn)(AttnArgs);
 
+struct Prefix {
+  KernelFn fn;
+  int threads;
+  size_t lds;
+};
+
+template <int D, int RT>
+Prefix prefix_of(bool aligned) {
+  using Gm = Geo<D, RT>;
+  return Prefix{aligned ? &spec_prefix_kernel<D, RT, true> : &spec_prefix_kernel<D, RT, false>, Gm::kThreads,
+                (size_t)Gm::kLds};
+}
+
 template <int D>
-KernelFn prefix_fn(int rt) {
+Prefix prefix_for(int rt, bool aligned) {
   switch (rt) {
-    case 1: return &spec_prefix_kernel<D, 1>;
-    case 2: return &spec_prefix_kernel<D, 2>;
-    case 3: return &spec_prefix_kernel<D, 3>;
-    case 4: return &spec_prefix_kernel<D, 4>;
-    default: return nullptr;
+    case 1: return prefix_of<D, 1>(aligned);
+    case 2: return prefix_of<D, 2>(aligned);
+    case 3: return prefix_of<D, 3>(aligned);
+    case 4: return prefix_of<D, 4>(aligned);
+    default: return Prefix{nullptr, 0, 0};
   }
 }
 
 std::mutex g_lds_mutex;
 std::unordered_set<const void*> g_lds_raised;
 
-int launch(KernelFn fn, dim3 grid, size_t smem, hipStream_t stream, const AttnArgs& a) {
+int launch(KernelFn fn, dim3 grid, int threads, size_t smem, hipStream_t stream, const AttnArgs& a) {
   void* args[] = {const_cast<AttnArgs*>(&a)};
   if (smem > kDefaultLds) {
     std::lock_guard<std::mutex> lock(g_lds_mutex);
@@ -578,7 +762,7 @@ int launch(KernelFn fn, dim3 grid, size_t smem, hipStream_t stream, const AttnAr
       g_lds_raised.insert(key);
     }
   }
-  if (hipLaunchKernel(reinterpret_cast<const void*>(fn), grid, dim3(kThreads), args, smem, stream) != hipSuccess)
+  if (hipLaunchKernel(reinterpret_cast<const void*>(fn), grid, dim3(threads), args, smem, stream) != hipSuccess)
     return QF_ERR_HIP;
   return QF_OK;
 }
@@ -590,6 +774,91 @@ size_t workspace_for(int B, int Q, int H, int HKV, int D, int S) {
   const size_t R = (size_t)Q * (H / HKV);
   const size_t n = (size_t)B * HKV * S * R * (D + 1) * sizeof(float);
   return (n + 255) / 256 * 256;
+}
+
+int run(const uint16_t* query, int64_t q_stride_tok, int64_t q_stride_head, const uint16_t* key_cache,
+        int64_t k_stride_block, int64_t k_stride_tok, int64_t k_stride_head, const uint16_t* value_cache,
+        int64_t v_stride_block, int64_t v_stride_tok, int64_t v_stride_head, const int32_t* block_table,
+        int64_t bt_stride, const int32_t* seq_lens, uint16_t* out, int64_t o_stride_tok, int64_t o_stride_head,
+        int num_reqs, int q_len, int num_heads, int num_kv_heads, int head_size, int page_size, float scale,
+        int num_splits, int min_chunk, int balanced, void* workspace, size_t workspace_bytes, void* stream) {
+  if (!query || !key_cache || !value_cache || !block_table || !seq_lens || !out) return QF_ERR_INVALID_ARG;
+  if (num_reqs < 1 || q_len < 1 || num_heads < 1 || num_kv_heads < 1 || page_size < 1 || num_splits < 1 ||
+      num_splits > 65535 || min_chunk < 1 || bt_stride < 0)
+    return QF_ERR_INVALID_ARG;
+  if (!(scale == scale)) return QF_ERR_INVALID_ARG;
+  if (num_heads % num_kv_heads) return QF_ERR_UNSUPPORTED;
+  const int G = num_heads / num_kv_heads;
+  const int R = q_len * G;
+  if (R > kMaxRows || page_size < QF_SPEC_ATTN_MIN_PAGE) return QF_ERR_UNSUPPORTED;
+  if (head_size != 64 && head_size != 128 && head_size != 256) return QF_ERR_UNSUPPORTED;
+  if ((int64_t)num_reqs * num_kv_heads > 65535 || (int64_t)num_reqs * q_len * num_heads > 0x7fffffff)
+    return QF_ERR_UNSUPPORTED;
+  const int64_t strides[] = {q_stride_tok, q_stride_head, k_stride_block, k_stride_tok, k_stride_head,
+                             v_stride_block, v_stride_tok, v_stride_head, o_stride_tok, o_stride_head};
+  for (int64_t s : strides)
+    if (s < 0 || s % 8) return QF_ERR_UNSUPPORTED;
+  // the prefix kernel keeps per-lane byte offsets of up to one stage of rows in 32 bits
+  if ((k_stride_tok > v_stride_tok ? k_stride_tok : v_stride_tok) * 2 * kKeyBlock >= ((int64_t)1 << 31))
+    return QF_ERR_UNSUPPORTED;
+  if (!aligned16(query) || !aligned16(key_cache) || !aligned16(value_cache) || !aligned16(out))
+    return QF_ERR_UNSUPPORTED;
+  if (balanced && (num_reqs > kMaxBalanced || num_splits < num_reqs)) return QF_ERR_UNSUPPORTED;
+  // split slots per kv head: one set a request, or one set shared by all
+  const int sets = balanced ? 1 : num_reqs;
+  const size_t part_bytes = workspace_for(sets, q_len, num_heads, num_kv_heads, head_size, num_splits);
+  const size_t need = part_bytes + (balanced ? QF_SPEC_ATTN_PLAN_BYTES : 0);
+  if (workspace == nullptr || workspace_bytes < need || !aligned16(workspace)) return QF_ERR_WORKSPACE;
+
+  AttnArgs a;
+  a.q = query;
+  a.sq_t = q_stride_tok;
+  a.sq_h = q_stride_head;
+  a.kc = key_cache;
+  a.sk_b = k_stride_block;
+  a.sk_t = k_stride_tok;
+  a.sk_h = k_stride_head;
+  a.vc = value_cache;
+  a.sv_b = v_stride_block;
+  a.sv_t = v_stride_tok;
+  a.sv_h = v_stride_head;
+  a.bt = block_table;
+  a.sbt = bt_stride;
+  a.seq_lens = seq_lens;
+  a.out = out;
+  a.so_t = o_stride_tok;
+  a.so_h = o_stride_head;
+  const size_t n_o = (size_t)sets * num_kv_heads * num_splits * R * head_size;
+  a.o_part = static_cast<float*>(workspace);
+  a.lse_part = a.o_part + n_o;
+  a.B = num_reqs;
+  a.Q = q_len;
+  a.H = num_heads;
+  a.HKV = num_kv_heads;
+  a.G = G;
+  a.R = R;
+  a.page = page_size;
+  a.splits = num_splits;
+  a.min_chunk = min_chunk;
+  a.qk_scale = scale * kLog2e;
+  a.by_g = divisor(G);
+  a.by_splits = divisor(num_splits);
+  a.by_page = divisor(page_size);
+  a.plan = balanced ? reinterpret_cast<int2*>(static_cast<uint8_t*>(workspace) + part_bytes) : nullptr;
+
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int rt = (R + 15) / 16;
+  Prefix pre;
+  KernelFn comb;
+  switch (head_size) {
+    case 64: pre = prefix_for<64>(rt, page_size % 16 == 0); comb = &spec_combine_kernel<64>; break;
+    case 128: pre = prefix_for<128>(rt, page_size % 16 == 0); comb = &spec_combine_kernel<128>; break;
+    default: pre = prefix_for<256>(rt, page_size % 16 == 0); comb = &spec_combine_kernel<256>; break;
+  }
+  if (pre.fn == nullptr) return QF_ERR_UNSUPPORTED;
+  int st = launch(pre.fn, dim3(num_splits, num_kv_heads, sets), pre.threads, pre.lds, s, a);
+  if (st != QF_OK) return st;
+  return launch(comb, dim3(num_reqs * q_len * num_heads, head_size / kCombSlice), kThreads, 0, s, a);
 }
 
 }  // namespace qfa
@@ -616,75 +885,27 @@ int qf_spec_attention(const uint16_t* query, int64_t q_stride_tok, int64_t q_str
                       int num_reqs, int q_len, int num_heads, int num_kv_heads, int head_size,
                       int page_size, float scale, int num_splits, int min_chunk,
                       void* workspace, size_t workspace_bytes, void* stream) {
-  if (!query || !key_cache || !value_cache || !block_table || !seq_lens || !out) return QF_ERR_INVALID_ARG;
-  if (num_reqs < 1 || q_len < 1 || num_heads < 1 || num_kv_heads < 1 || page_size < 1 || num_splits < 1 ||
-      num_splits > 65535 || min_chunk < 1 || bt_stride < 0)
-    return QF_ERR_INVALID_ARG;
-  if (!(scale == scale)) return QF_ERR_INVALID_ARG;
-  if (num_heads % num_kv_heads) return QF_ERR_UNSUPPORTED;
-  const int G = num_heads / num_kv_heads;
-  const int R = q_len * G;
-  if (R > kMaxRows || page_size < QF_SPEC_ATTN_MIN_PAGE) return QF_ERR_UNSUPPORTED;
-  if (head_size != 64 && head_size != 128 && head_size != 256) return QF_ERR_UNSUPPORTED;
-  if ((int64_t)num_reqs * num_kv_heads > 65535 || (int64_t)num_reqs * q_len * num_heads > 0x7fffffff)
-    return QF_ERR_UNSUPPORTED;
-  const int64_t strides[] = {q_stride_tok, q_stride_head, k_stride_block, k_stride_tok, k_stride_head,
-                             v_stride_block, v_stride_tok, v_stride_head, o_stride_tok, o_stride_head};
-  for (int64_t s : strides)
-    if (s < 0 || s % 8) return QF_ERR_UNSUPPORTED;
-  // the prefix kernel keeps per-lane byte offsets of up to one stage of rows in 32 bits
-  if ((k_stride_tok > v_stride_tok ? k_stride_tok : v_stride_tok) * 2 * kKeyBlock >= ((int64_t)1 << 31))
-    return QF_ERR_UNSUPPORTED;
-  if (!aligned16(query) || !aligned16(key_cache) || !aligned16(value_cache) || !aligned16(out))
-    return QF_ERR_UNSUPPORTED;
-  const size_t need = workspace_for(num_reqs, q_len, num_heads, num_kv_heads, head_size, num_splits);
-  if (workspace == nullptr || workspace_bytes < need || !aligned16(workspace)) return QF_ERR_WORKSPACE;
+  return run(query, q_stride_tok, q_stride_head, key_cache, k_stride_block, k_stride_tok, k_stride_head, value_cache,
+             v_stride_block, v_stride_tok, v_stride_head, block_table, bt_stride, seq_lens, out, o_stride_tok,
+             o_stride_head, num_reqs, q_len, num_heads, num_kv_heads, head_size, page_size, scale, num_splits,
+             min_chunk, 0, workspace, workspace_bytes, stream);
+}
 
-  AttnArgs a;
-  a.q = query;
-  a.sq_t = q_stride_tok;
-  a.sq_h = q_stride_head;
-  a.kc = key_cache;
-  a.sk_b = k_stride_block;
-  a.sk_t = k_stride_tok;
-  a.sk_h = k_stride_head;
-  a.vc = value_cache;
-  a.sv_b = v_stride_block;
-  a.sv_t = v_stride_tok;
-  a.sv_h = v_stride_head;
-  a.bt = block_table;
-  a.sbt = bt_stride;
-  a.seq_lens = seq_lens;
-  a.out = out;
-  a.so_t = o_stride_tok;
-  a.so_h = o_stride_head;
-  const size_t n_o = (size_t)num_reqs * num_kv_heads * num_splits * R * head_size;
-  a.o_part = static_cast<float*>(workspace);
-  a.lse_part = a.o_part + n_o;
-  a.B = num_reqs;
-  a.Q = q_len;
-  a.H = num_heads;
-  a.HKV = num_kv_heads;
-  a.G = G;
-  a.R = R;
-  a.page = page_size;
-  a.splits = num_splits;
-  a.min_chunk = min_chunk;
-  a.qk_scale = scale * kLog2e;
-
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const int rt = (R + 15) / 16;
-  KernelFn pre = nullptr, comb = nullptr;
-  size_t lds = 0;
-  switch (head_size) {
-    case 64: pre = prefix_fn<64>(rt); comb = &spec_combine_kernel<64>; lds = Geo<64>::kLds; break;
-    case 128: pre = prefix_fn<128>(rt); comb = &spec_combine_kernel<128>; lds = Geo<128>::kLds; break;
-    default: pre = prefix_fn<256>(rt); comb = &spec_combine_kernel<256>; lds = Geo<256>::kLds; break;
-  }
-  if (pre == nullptr) return QF_ERR_UNSUPPORTED;
-  int st = launch(pre, dim3(num_splits, num_reqs * num_kv_heads), lds, s, a);
-  if (st != QF_OK) return st;
-  return launch(comb, dim3(num_reqs * q_len * num_heads, head_size / kCombSlice), 0, s, a);
+int qf_spec_attention_balanced(const uint16_t* query, int64_t q_stride_tok, int64_t q_stride_head,
+                               const uint16_t* key_cache, int64_t k_stride_block, int64_t k_stride_tok,
+                               int64_t k_stride_head,
+                               const uint16_t* value_cache, int64_t v_stride_block, int64_t v_stride_tok,
+                               int64_t v_stride_head,
+                               const int32_t* block_table, int64_t bt_stride,
+                               const int32_t* seq_lens,
+                               uint16_t* out, int64_t o_stride_tok, int64_t o_stride_head,
+                               int num_reqs, int q_len, int num_heads, int num_kv_heads, int head_size,
+                               int page_size, float scale, int total_splits, int min_chunk,
+                               void* workspace, size_t workspace_bytes, void* stream) {
+  return run(query, q_stride_tok, q_stride_head, key_cache, k_stride_block, k_stride_tok, k_stride_head, value_cache,
+             v_stride_block, v_stride_tok, v_stride_head, block_table, bt_stride, seq_lens, out, o_stride_tok,
+             o_stride_head, num_reqs, q_len, num_heads, num_kv_heads, head_size, page_size, scale, total_splits,
+             min_chunk, 1, workspace, workspace_bytes, stream);
 }
 
 }  // extern "C"

@@ -18,12 +18,15 @@ MAX_ROWS = 64     # QF_SPEC_ATTN_MAX_ROWS
 MIN_PAGE = 16     # QF_SPEC_ATTN_MIN_PAGE
 KEY_BLOCK = 32    # QF_SPEC_ATTN_KEY_BLOCK
 HEAD_SIZES = (64, 128, 256)
+PLAN_BYTES = 512   # QF_SPEC_ATTN_PLAN_BYTES
+MAX_BALANCED = 64  # requests of qf_spec_attention_balanced
 
 # Every symbol include/qf_spec_attn.h declares.
 EXPORTS = (
     "qf_spec_attn_abi_version",
     "qf_spec_attn_workspace_bytes",
     "qf_spec_attention",
+    "qf_spec_attention_balanced",
 )
 
 _lib: ctypes.CDLL | None = None
@@ -53,6 +56,8 @@ def load() -> ctypes.CDLL:
                                     i32, i32, i32, i32, i32, i32, f32, i32, i32,
                                     p, sz, p]
     L.qf_spec_attention.restype = i32
+    L.qf_spec_attention_balanced.argtypes = L.qf_spec_attention.argtypes
+    L.qf_spec_attention_balanced.restype = i32
     v = L.qf_spec_attn_abi_version()
     if v != ABI_VERSION:
         raise ImportError(f"{LIB_PATH}: ABI version {v}, expected {ABI_VERSION}")

@@ -104,15 +104,21 @@ def gqa_packed_spec_attention(query, key_cache, value_cache, out, seq_lens, bloc
     if query.shape[0] < B * Q or out.shape[0] < B * Q or seq_lens.numel() < B or block_table.shape[0] < B:
         raise ValueError("batch tensors are smaller than num_reqs * Q")
     page = key_cache.shape[1]
+    L = AL.load()
+    attention, sets = L.qf_spec_attention, B
     if num_splits is None:
         num_splits = auto_num_splits(query.device, B, num_kv_heads)
-    L = AL.load()
-    ws_bytes = AL.workspace_bytes(B, Q, H, num_kv_heads, D, num_splits)
+        if 1 < B <= AL.MAX_BALANCED:  # one set of split slots a kv head, given out to the requests by length
+            attention, sets = L.qf_spec_attention_balanced, 1
+            num_splits = max(B, auto_num_splits(query.device, 1, num_kv_heads))
+    ws_bytes = AL.workspace_bytes(sets, Q, H, num_kv_heads, D, num_splits)
     if ws_bytes == 0:
         raise ValueError("invalid attention sizes")
+    if sets != B:
+        ws_bytes += AL.PLAN_BYTES
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=query.device)
     stream = torch.cuda.current_stream(query.device).cuda_stream
-    rc = L.qf_spec_attention(
+    rc = attention(
         query.data_ptr(), query.stride(0), query.stride(1),
         key_cache.data_ptr(), key_cache.stride(0), key_cache.stride(1), key_cache.stride(2),
         value_cache.data_ptr(), value_cache.stride(0), value_cache.stride(1), value_cache.stride(2),

@@ -90,11 +90,46 @@ def test_split_spanning_several_table_windows():
     _check(inp, _run(inp, num_splits=1), "windows page=16 splits=1")
 
 
+@pytest.mark.parametrize("D,HKV,G,Q,page,lens", [
+    (128, 4, 8, 5, 16, [9005, 7672, 6339, 5006, 3673, 2340]),  # 3 row tiles; the splits go by length
+    (256, 2, 6, 3, 800, [5003, 3, 64 + 3, 65 + 3, 2, 1, 2000]),  # no prefix, one stage, one stage and a position
+    (256, 1, 8, 8, 24, [3000, 17, 700]),                       # 4 row tiles, pages that cut key tiles
+    (256, 2, 6, 8, 17, [1111, 900]),                           # 3 row tiles
+    (128, 8, 8, 8, 16, [4200, 77, 129, 128 + 8]),              # 4 row tiles, 4 wavefronts
+    (128, 2, 1, 2, 64, [131, 127, 5000]),                      # 1 row tile
+    (64, 4, 8, 4, 17, [3001, 16, 260]),                        # 2 row tiles, every other one a wavefront
+    (64, 2, 7, 7, 32, [70, 8000]),                             # 4 row tiles
+    (64, 1, 2, 2, 16, [1 + 40 * i for i in range(64)]),            # the most requests
+])
+def test_balanced_batches(D, HKV, G, Q, page, lens):
+    """Ragged batches through the balanced splits; every cache row that no query may see holds NaN, and the later
+    positions score higher, so that the exponent references move stage after stage."""
+    inp = A.gen_spec_inputs(max(lens), Q, len(lens), H=G * HKV, HKV=HKV, D=D, page=page, seed=D + Q + page, lens=lens)
+    nan = np.ones(inp.kv.shape[:1] + inp.kv.shape[2:3], dtype=bool)  # [page id, row]
+    for b, n in enumerate(lens):
+        pos = np.arange(n)
+        nan[inp.block_table[b, pos // page], pos % page] = False
+        blk, off = inp.block_table[b, pos // page], pos % page
+        grow = (1.0 + 6.0 * pos / max(lens))[:, None, None]
+        k = A.bf16_bits_to_f32(inp.kv[blk, :, off, :D]) * grow
+        inp.kv[blk, :, off, :D] = A.bf16_bits_from_f32(k.astype(np.float32))
+    kv_clean = inp.kv.copy()
+    inp.kv.transpose(0, 2, 1, 3)[nan] = 0x7FC0
+    out = _run(inp)
+    inp.kv[:] = kv_clean
+    _check(inp, out, f"balanced D={D} HKV={HKV} G={G} Q={Q} page={page} lens={lens[:7]}")
+
+
 def test_rows_that_see_nothing_are_zero():
     inp = A.gen_spec_inputs(0, 4, 3, seed=5, lens=[1, 2, 4])
     out = _run(inp)
     _check(inp, out, "short requests")
     assert np.all(out[0:3] == 0) and np.all(out[4:6] == 0)
+
+
+def test_empty_request_in_a_batch_is_zero():
+    inp = A.gen_spec_inputs(300, 3, 2, seed=6, lens=[0, 303])
+    assert np.all(_run(inp)[:3] == 0)
 
 
 def test_deterministic():

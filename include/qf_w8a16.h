@@ -129,7 +129,9 @@ const char* qf_status_string(int status);
  * shape is not served (M < 1, M > 16 on row-major weights, N < 1, K % 64 != 0, unknown layout),
  * mirroring pick_config() returning None.  M > 16 on TILED weights gets QF_KERNEL_MFMA_WIDE (the
  * reference sends M > 16 to its W8A8 fallback, plugin/qwen_fastpath/patches.py:99-100, which cannot
- * read the TILED image).  Host-only; touches no device. */
+ * read the TILED image).  On row-major weights at 2 <= M <= 16 an automatic qf_w8a16_gemm may run the
+ * library's row stream kernel instead, which has no explicit form, within this configuration's
+ * workspace (its sums differ in order only).  Host-only; touches no device. */
 int qf_w8a16_pick_config(int M, int N, int K, int layout, qf_w8a16_config* cfg);
 
 /* Bytes of device workspace qf_w8a16_gemm needs for this call (0 when split_k == 1): arrival

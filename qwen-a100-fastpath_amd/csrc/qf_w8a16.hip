@@ -230,6 +230,23 @@ __device__ __forceinline__ uint64_t argmax_key(float v, int i) {
 // s_waitcnt immediate (gfx9 encoding) that waits for vmcnt == 0 and leaves expcnt / lgkmcnt free.
 constexpr int kWaitVmcnt0 = 0x0F70;
 
+constexpr int kNonTemporalAux = 2;  // cache-policy operand of a direct-to-LDS load: read once
+
+typedef const void __attribute__((address_space(1)))* glb_ptr_t;
+typedef void __attribute__((address_space(3)))* lds_ptr_t;
+
+// s_waitcnt with vmcnt = n (0..63) and the other counters unconstrained.
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+  static_assert(N >= 0 && N < 64, "vmcnt range");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
+}
+
+// 32-bit LDS address of a pointer into the workgroup's LDS
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
+}
+
 // Workgroup barrier that orders LDS accesses only.  __syncthreads() also orders global memory, for
 // which it waits until every global load of the wavefront has returned: issued after a prefetch,
 // that drains the prefetch before the first step.  Here the global loads stay in flight.
@@ -1059,6 +1076,197 @@ __global__ void __launch_bounds__(W * kWave) w8a16_stream_xreg_kernel(const Gemm
 }
 
 // ---------------------------------------------------------------------------------------------
+// Row stream kernel: automatic calls on the row-major layout, 2 <= M <= 16 (rows_plan).
+//
+// An MFMA fragment takes 16 rows x 64 k, so a wavefront that loads it straight from row-major weights asks for sixteen
+// 64-byte halves of cache lines (gate_up 34816 x 5120 at M = 11: 52.5 us with its second pass).  Here the weights go
+// global -> LDS by direct-to-LDS copies whose lanes cover whole 128-byte lines (8 rows x 128 k an instruction), and the
+// fragments are read from there: the copies write linearly, so the 16-byte piece of row n that lands at position p of
+// its 128 bytes is piece p ^ ((n >> 1) & 7), which spreads a fragment read's 16 rows over the banks.
+//
+// The grid is (runs of 16-row tiles, K splits), about one workgroup a CU; a workgroup's 8 wavefronts interleave over the
+// 128-k pairs of steps of its K range: wavefront v takes the pairs v, v + 8, ... of every tile, holds their x fragments
+// in registers (4 a pair, S pairs at most, zero past the range) and streams its pairs, tile after tile, through two
+// 2 KiB LDS slots of its own, one in flight while the other is multiplied: no barrier before the sums.  Two slots a
+// wavefront (32 KiB a CU in flight) measured best of 2, 3, 4 and 6; the x requests go out before the weights (level
+// with after); 8-byte fragment granules, which halve the lines of an x request, are level too.
+// LINES: the rows start on 128-byte lines, so no line is read twice and the copies bypass reuse (non-temporal: gate_up
+// M = 11 32.5 against 35.8 us); rows that do not (K an odd number of steps) share each line between two wavefronts' pairs
+// and keep it cached (N = 6539, K = 10944, M = 14: 22.2 against 23.0 us).
+// Sums in a fixed order as in the stream kernel: each wavefront parks its partial tile in LDS, wavefront v then adds
+// the 8 partials of tiles v, v + 8, ... in wavefront order; with a K split the last workgroup of a run adds the splits
+// in split order (the MFMA kernel's device-scope partials and arrival counter).
+// Bound by memory on wide weights (gate_up M = 5 31.2 us, 5.7 TB/s, against 43.0 on the MFMA kernel; M = 11 32.5
+// against 52.5; M = 16 34.0 against 49.9), by the x requests' L2 traffic, the run's unevenness and the sums on narrow
+// ones (M = 11: qkv 14.6 against 20.3, o_proj 13.8 against 15.2, down 22.8 against 24.7).  Over 90 shapes of 512 to
+// 40000 channels, K 512 to 17920 and M 2 to 16 drawn at random it takes 0.75 of the time of the kernels before it, at
+// worst 1.07 (an odd K whose pairs do not share out over the wavefronts).
+// ---------------------------------------------------------------------------------------------
+constexpr int kRowsWaves = 8;
+constexpr int kRowsSlots = 2;
+constexpr int kRowsMaxPairs = 10;          // pairs a wavefront: 160 registers of x fragments
+constexpr int kRowsPairBytes = 2 * kTileN * kStepK;
+constexpr int kRowsRing = kRowsWaves * kRowsSlots * kRowsPairBytes;
+
+template <int S, bool LINES>
+__global__ void __launch_bounds__(kRowsWaves * kWave) __attribute__((amdgpu_waves_per_eu(2, 2)))
+    w8a16_rows_kernel(const GemmArgs a) {
+  extern __shared__ __align__(16) uint8_t smem[];
+  __shared__ int last_arrival;
+  constexpr int W = kRowsWaves, D = kRowsSlots;
+  constexpr int kAux = LINES ? kNonTemporalAux : 0;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int v = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int g = lane >> 4;
+  const int r = lane & 15;
+  const int ntiles = a.n_pad / kTileN;
+  const int t0 = (int)(((int64_t)blockIdx.x * ntiles) / gridDim.x);
+  const int nt = (int)(((int64_t)(blockIdx.x + 1) * ntiles) / gridDim.x) - t0;  // >= 1: at most ntiles columns
+  // The split's pairs [p_begin, p_end): splits start on whole pairs, so that a pair is a 128-byte line where the rows
+  // are (a split of 91 steps, its lines cut in two, took down 5120 x 17408 from 22 to 27 us).
+  int p_begin, p_end;
+  split_range(blockIdx.y, a.split_k, (a.ksteps + 1) / 2, p_begin, p_end);
+  const int mine = p_end - p_begin > v ? (p_end - p_begin - v + W - 1) / W : 0;  // at most S
+  uint8_t* const ring = smem + v * D * kRowsPairBytes;
+  f32x4_t* const part = reinterpret_cast<f32x4_t*>(smem + kRowsRing);  // [nt][W][64 lanes]
+
+  if (mine > 0) {  // uniform
+    // x fragments of the wavefront's pairs: lane (g, r) holds x[min(r, M - 1)][64 s + 16 g .. + 15] of both steps
+    const uint16_t* xp = a.x + (int64_t)min(r, a.M - 1) * a.ldx + 16 * g;
+    u32x4_t xf[S][4];
+#pragma unroll
+    for (int p = 0; p < S; ++p)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int s = min(2 * (p_begin + v + p * W) + h, a.ksteps - 1);
+        const u32x4_t* q = reinterpret_cast<const u32x4_t*>(xp + (int64_t)s * kStepK);
+        xf[p][2 * h] = q[0];
+        xf[p][2 * h + 1] = q[1];
+      }
+    __builtin_amdgcn_sched_barrier(0);
+
+    // The copy cursor: pair cp of tile ct, into slot ci % D.  Lane l of a pair's two copies takes row l / 8 (+ 8),
+    // 16-byte position l % 8.  Rows past N read the last row; past the last pair the cursor goes round the last tile
+    // again (in-bounds re-reads into slots that are read no more), so that every copy is made and counted.
+    const int lrow = lane >> 3;
+    const int piece = (lane & 7) ^ (lrow >> 1);  // rows 8 .. 15 flip piece bit 2 besides
+    int ct = 0, cp = 0, ci = 0;
+    const int8_t *row0, *row1;
+    auto set_rows = [&]() {
+      const int n = (t0 + ct) * kTileN + lrow;
+      row0 = a.w + (int64_t)min(n, a.N - 1) * a.ldw;
+      row1 = a.w + (int64_t)min(n + 8, a.N - 1) * a.ldw;
+    };
+    set_rows();
+    auto copy = [&]() {
+      const int pair = p_begin + v + cp * W;
+      uint8_t* dst = ring + (ci % D) * kRowsPairBytes;
+      int q0 = piece, q1 = piece ^ 4;
+      if (2 * pair + 1 == a.ksteps) {  // an odd K's last pair has one step: its bytes twice (the second's x are 0)
+        q0 &= 3;
+        q1 &= 3;
+      }
+      const int64_t k = (int64_t)pair * (2 * kStepK);
+      __builtin_amdgcn_global_load_lds((glb_ptr_t)(row0 + k + q0 * 16), (lds_ptr_t)dst, 16, 0, kAux);
+      __builtin_amdgcn_global_load_lds((glb_ptr_t)(row1 + k + q1 * 16), (lds_ptr_t)(dst + 1024), 16, 0, kAux);
+      ++ci;
+      if (++cp == mine) {
+        cp = 0;
+        if (ct < nt - 1) {
+          ++ct;
+          set_rows();
+        }
+      }
+    };
+#pragma unroll
+    for (int d = 0; d < D; ++d) copy();
+    wait_vmcnt<2 * D>();  // the x fragments have landed
+#pragma unroll
+    for (int p = 0; p < S; ++p)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        if (2 * (p_begin + v + p * W) + h >= a.ksteps) xf[p][2 * h] = xf[p][2 * h + 1] = (u32x4_t){0u, 0u, 0u, 0u};
+
+    // fragment addresses of a slot: row r, piece g of the first step, piece 4 + g of the second
+    const uint32_t f0 = lds_addr(ring) + r * 128 + ((g ^ ((r >> 1) & 7)) << 4);
+    const uint32_t f1 = lds_addr(ring) + r * 128 + (((4 + g) ^ ((r >> 1) & 7)) << 4);
+    uint32_t slot = 0;
+    for (int t = 0; t < nt; ++t) {
+      f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int p = 0; p < S; ++p) {
+        if (p < mine) {  // uniform
+          wait_vmcnt<2 * (D - 1)>();  // this pair's copies have landed
+          // Read by inline assembly: the compiler would wait for every copy in flight before a plain LDS read.
+          u32x4_t w0, w1;
+          asm volatile("ds_read_b128 %0, %1" : "=v"(w0) : "v"(f0 + slot));
+          asm volatile("ds_read_b128 %0, %1" : "=v"(w1) : "v"(f1 + slot));
+          asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(w0), "+v"(w1) : : "memory");
+          copy();  // the reads have returned: into the slot they read
+          slot = slot == (D - 1) * kRowsPairBytes ? 0 : slot + kRowsPairBytes;
+          bf16x8_t b0, b1;
+          dequant16(w0, b0, b1);
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b0, __builtin_bit_cast(bf16x8_t, xf[p][0]), acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b1, __builtin_bit_cast(bf16x8_t, xf[p][1]), acc, 0, 0, 0);
+          dequant16(w1, b0, b1);
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b0, __builtin_bit_cast(bf16x8_t, xf[p][2]), acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b1, __builtin_bit_cast(bf16x8_t, xf[p][3]), acc, 0, 0, 0);
+        }
+      }
+      part[(t * W + v) * kWave + lane] = acc;
+    }
+    wait_vmcnt<0>();  // no copy lands once the workgroup's LDS is given back
+  } else {
+    for (int t = 0; t < nt; ++t) part[(t * W + v) * kWave + lane] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  }
+  __syncthreads();
+  // Lane (g, r) holds C[n = tile * 16 + 4 g + i][m = r], i = 0..3, in each partial.
+  const int64_t plane = (int64_t)a.M * a.n_pad;
+  for (int t = v; t < nt; t += W) {
+    f32x4_t sum = part[(t * W) * kWave + lane];
+#pragma unroll
+    for (int u = 1; u < W; ++u) sum += part[(t * W + u) * kWave + lane];
+    const int n = (t0 + t) * kTileN + 4 * g;
+    if (a.split_k == 1) {
+      if (r < a.M && n < a.N)
+        store_out4(a.y, a.ldy, a.out_f32, a.vec_out, r, n, min(4, a.N - n), sum * load_scale4(a.scale, a.N, n));
+    } else if (r < a.M) {
+      float* dst = a.partial + (int64_t)blockIdx.y * plane + (int64_t)r * a.n_pad + n;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) __hip_atomic_store(dst + i, sum[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  if (a.split_k == 1) return;
+  // Last arrival, ordered as in w8a16_mfma_kernel.
+  __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const unsigned prev = __hip_atomic_fetch_add(a.counters + blockIdx.x * a.counter_stride, 1u, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT);
+    last_arrival = prev == (unsigned)(a.split_k - 1);
+  }
+  __syncthreads();
+  if (!last_arrival) return;
+  for (int t = v; t < nt; t += W) {
+    const int n = (t0 + t) * kTileN + 4 * g;
+    if (r < a.M && n < a.N) {
+      float* src = a.partial + (int64_t)r * a.n_pad + n;
+      f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < a.split_k; ++j) {
+        f32x4_t p;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          p[i] = __hip_atomic_load(src + j * plane + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        sum = j == 0 ? p : sum + p;
+      }
+      store_out4(a.y, a.ldy, a.out_f32, a.vec_out, r, n, min(4, a.N - n), sum * load_scale4(a.scale, a.N, n));
+    }
+  }
+  if (threadIdx.x == 0)
+    __hip_atomic_store(a.counters + blockIdx.x * a.counter_stride, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// ---------------------------------------------------------------------------------------------
 // Wide-M MFMA kernel, TILED layout: M > 16 (prefill chunks, long verification batches).
 //
 // A workgroup owns WN * NT 16-row weight tiles over the whole K range (one wavefront per NT tiles,
@@ -1667,22 +1875,12 @@ __global__ void __launch_bounds__(WN * kWave) w8a8_wide_kernel(const GemmArgs a)
 // 256-byte row pieces (the MFMA layout alone would store 16 rows x 32 bytes per instruction: gate_up
 // M = 2048 406 -> 379 us); fp32 output or rows without 16-byte alignment store from the registers.
 // ---------------------------------------------------------------------------------------------
-typedef const void __attribute__((address_space(1)))* glb_ptr_t;
-typedef void __attribute__((address_space(3)))* lds_ptr_t;
-
 constexpr int kW8A8TileStages = 4;
 constexpr int kW8A8TileRows = 256;                        // tokens per workgroup
 constexpr int kW8A8TileTiles = 16;                        // 16-channel weight tiles per workgroup
 constexpr int kW8A8TileStageBytes = 32 * 1024;            // 16 weight + 16 activation fragments
 constexpr int kW8A8TileLds = kW8A8TileStages * kW8A8TileStageBytes;
 constexpr int kW8A8TileMaxSplit = 8;                      // K splits of the tile kernel (fused reduction)
-
-// s_waitcnt with vmcnt = n (0..63) and the other counters unconstrained.
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
-}
 
 // Workgroup tile shapes: FA weight fragments by FB activation fragments a wavefront, 8 wavefronts in 2
 // channel x 4 token groups, so 32 FA channels x 64 FB tokens a workgroup: (8, 4) is the 256 x 256 main
@@ -2676,6 +2874,19 @@ KernelFn select_stream_xreg(int waves, int depth, int ksteps) {
   return nullptr;
 }
 
+// The row stream kernel for `pairs` pairs a wavefront.
+template <bool LINES>
+KernelFn rows_by_pairs(int pairs) {
+  if (pairs <= 1) return &w8a16_rows_kernel<1, LINES>;
+  if (pairs <= 2) return &w8a16_rows_kernel<2, LINES>;
+  if (pairs <= 3) return &w8a16_rows_kernel<3, LINES>;
+  if (pairs <= 4) return &w8a16_rows_kernel<4, LINES>;
+  if (pairs <= 5) return &w8a16_rows_kernel<5, LINES>;
+  if (pairs <= 6) return &w8a16_rows_kernel<6, LINES>;
+  if (pairs <= 8) return &w8a16_rows_kernel<8, LINES>;
+  return pairs <= kRowsMaxPairs ? &w8a16_rows_kernel<kRowsMaxPairs, LINES> : nullptr;
+}
+
 // Compute units of the current device (the stream kernel's grid), cached per device; 256 (an MI355X)
 // when no device is visible, so that host-only configuration queries still answer.
 constexpr int kMaxCuDevices = 64;
@@ -3138,6 +3349,43 @@ int launch(KernelFn fn, dim3 grid, dim3 block, size_t smem, hipStream_t stream, 
   return QF_OK;
 }
 
+// The row stream kernel's launch: `columns` runs of at most `run` tiles, by `split` ranges of K, `pairs` pairs of
+// k-steps for the busiest wavefront; columns 0 where it does not serve the shape.
+struct RowsPlan {
+  int columns, run, split, pairs;
+};
+
+// The least time of the busiest wavefront, in pairs (tiles of a run times pairs a tile), over the splits up to max_split
+// (the planes that the caller's workspace holds) that run in one round of workgroups, one a CU, with a run's partial
+// tiles in LDS (15 tiles: up to 61440 channels; a vocabulary keeps the MFMA kernel, whose sums its fused argmax shares);
+// a split costs about a pair and a half, its partials' round trip: qkv 10240 x 5120
+// at M = 5 3 x 5 unsplit 13.1 us, 5 x 3 in two splits 14.8; o_proj 5120 x 8192 2 x 8 unsplit 13.8, 3 x 4 in two 13.6.
+RowsPlan rows_plan(int N, int K, int max_split) {
+  const int all_pairs = (K / kStepK + 1) / 2;
+  const int ntiles = round_up16(N) / kTileN;
+  const int cus = device_cus();
+  constexpr int kMaxRun = (int)((kMaxLds - kRowsRing) / (kRowsWaves * kWave * sizeof(f32x4_t)));
+  RowsPlan best{0, 0, 0, 0};
+  double best_cost = 0;
+  for (int split = 1; split <= std::min(max_split, all_pairs); ++split) {
+    RowsPlan p;
+    p.split = split;
+    p.pairs = ceil_div(ceil_div(all_pairs, split), kRowsWaves);
+    if (p.pairs > kRowsMaxPairs) continue;
+    const int columns = std::max(1, cus / split);
+    p.run = ceil_div(ntiles, columns);
+    if (p.run > kMaxRun) continue;
+    p.columns = ceil_div(ntiles, p.run);
+    if (split > 1 && (size_t)p.columns * 4 > QF_W8A16_COUNTER_BYTES) continue;  // an arrival counter a run
+    const double cost = (double)p.run * p.pairs + (split > 1 ? 1.0 + 0.25 * split : 0.0);
+    if (best.columns == 0 || cost < best_cost) {
+      best = p;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
 // Words between the arrival counters of n workgroup groups: spread over the counter prefix (up to 1 KiB apart),
 // since atomics on nearby addresses share a memory channel (measured on the fused argmax: 64 slots 64 bytes apart
 // cost 11 us on 9496 workgroups, 1 KiB apart about 3).
@@ -3213,6 +3461,19 @@ int run_gemm(const uint16_t* x, int64_t ldx, const int8_t* w, int64_t ldw, int l
   if (c.kernel == QF_KERNEL_MFMA_WIDE) wide_groups(M, a.groups, a.group_rows);
 
   const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  // Row-major weights at 2 or more tokens, automatic calls: whole-line copies (M = 1: the GEMV's row reads stay ahead on
+  // narrow N, qkv 11.9 against 12.6 us; the fused argmax and the normalising GEMM are epilogues of the other kernels).
+  if (layout == QF_LAYOUT_ROWMAJOR && M >= 2 && am == nullptr && norm_eps == nullptr &&
+      (cfg == nullptr || cfg->kernel == QF_KERNEL_AUTO)) {
+    const RowsPlan p = rows_plan(N, K, c.split_k);
+    if (p.columns > 0) {
+      a.split_k = p.split;
+      a.counter_stride = counter_stride_for(p.columns);
+      const bool lines = ldw % 128 == 0 && (reinterpret_cast<uintptr_t>(w) & 127) == 0;
+      return launch(lines ? rows_by_pairs<true>(p.pairs) : rows_by_pairs<false>(p.pairs), dim3(p.columns, p.split), dim3(kRowsWaves * kWave),
+                    (size_t)kRowsRing + (size_t)p.run * kRowsWaves * kWave * sizeof(f32x4_t), s, a);
+    }
+  }
   const dim3 grid = c.kernel == QF_KERNEL_MFMA_WIDE ? dim3(workgroups(c, N) * a.groups * c.split_k)
                                                     : dim3(workgroups(c, N), c.split_k);
   const dim3 block(c.waves * kWave);

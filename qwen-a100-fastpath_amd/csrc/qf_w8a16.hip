@@ -1880,6 +1880,14 @@ constexpr int kW8A8TileRows = 256;                        // tokens per workgrou
 constexpr int kW8A8TileTiles = 16;                        // 16-channel weight tiles per workgroup
 constexpr int kW8A8TileStageBytes = 32 * 1024;            // 16 weight + 16 activation fragments
 constexpr int kW8A8TileLds = kW8A8TileStages * kW8A8TileStageBytes;
+// Past 12 token blocks the tiles run in bands of 4 channel blocks, channel fastest: the 32 workgroups an XCD
+// runs at once then cover 8 token blocks by 4 channel blocks (12 blocks to fetch) instead of all the tokens
+// of 2 channel blocks (18 at M = 4096, 33 at M = 8192).  TILED, plain order against bands: gate_up M = 4096
+// 612.6 -> 594.0 us, M = 8192 1236 -> 1147; down M = 4096 305.1 -> 294.1; o_proj M = 4096 148.9 -> 144.4;
+// qkv M = 8192 359.5 -> 339.9.  At 12 blocks (M = 3072) both orders measure the same (460.4 and 460.7 on
+// gate_up), and up to 8 the plain order already covers 8 x 4.  Bands of 2, 3, 6 and 8 were within 2% of 4.
+constexpr int kW8A8TileBand = 4;
+constexpr int kW8A8TileBandRows = 12;
 constexpr int kW8A8TileMaxSplit = 8;                      // K splits of the tile kernel (fused reduction)
 
 // Workgroup tile shapes: FA weight fragments by FB activation fragments a wavefront, 8 wavefronts in 2
@@ -1918,7 +1926,8 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   const int ntiles = a.n_pad / kTileN;
   const int mblocks = (a.M + T::rows - 1) / T::rows;
   // The hardware hands workgroup i to XCD i % kXcds; consecutive logical blocks share an XCD, so the
-  // token blocks of one channel block run together and share its weights in that XCD's L2.
+  // token blocks of one channel block (of a band of them, past kW8A8TileBandRows) run together and share its
+  // weights in that XCD's L2.
   int l = xcd_major(blockIdx.x, gridDim.x);
   // split_k > 1: the grid is split_k copies of the tile grid, copy `split` computing k-steps
   // [s_begin, s_end) of every tile.
@@ -1928,8 +1937,17 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   int s_begin = 0, s_end = a.ksteps;
   if (a.split_k > 1) split_range(split, a.split_k, a.ksteps, s_begin, s_end);
   const int nsteps = s_end - s_begin;  // >= 1: split_k <= ksteps
-  const int tile0 = (l / mblocks) * T::tiles;
-  const int m0 = (l % mblocks) * T::rows;
+  int nb = l / mblocks, mb = l % mblocks;
+  if (mblocks > kW8A8TileBandRows) {
+    const int nblocks = tiles_grid / mblocks;
+    const int band = l / (kW8A8TileBand * mblocks);
+    const int width = min(kW8A8TileBand, nblocks - band * kW8A8TileBand);
+    const int q = l - band * kW8A8TileBand * mblocks;
+    nb = band * kW8A8TileBand + q % width;
+    mb = q / width;
+  }
+  const int tile0 = nb * T::tiles;
+  const int m0 = mb * T::rows;
   const int ksteps = a.ksteps;
 
   // Wavefront w copies fragments CP w .. CP w + CP - 1 of the stage: the T::tiles weight fragments first, then
@@ -3769,7 +3787,8 @@ int w8a8_plan(int M, int N, int K, int layout, const qf_w8a16_config& c, W8a8Lau
     // number 128 to 256 (reduce 0), else (or with reduce 2) the wide kernel.  Token-tiled activations,
     // gate_up M = 2048 (1024 workgroups, 2048 channels left): 304.5 us, 323.1 with the wide kernel's tail,
     // 316.3 in one launch; qkv M = 2048: 92.1 / 112.9 / 111.9 us.  Past a quarter round one launch is
-    // faster (gate_up M = 4096, 128 past 2048: 600 us, 613 with two rounds of 128 x 128 workgroups).
+    // faster (gate_up M = 4096, 128 past 2048, in the plain tile order: 600 us, 613 with two rounds of 128 x 128
+    // workgroups).
     const int nblocks = ceil_div(n_pad / kTileN, kW8A8TileTiles);
     const int mblocks = ceil_div(M, kW8A8TileRows);
     const int64_t twgs = (int64_t)nblocks * mblocks;

@@ -359,6 +359,24 @@ def test_w8a8_tile_kernel_tail_split(M, N, K):
                         assert torch.isnan(y[:, N:].float()).all(), case
 
 
+@pytest.mark.parametrize("M,N", [(3329, 1288), (3073, 264), (3072, 1288)])
+@pytest.mark.parametrize("split,red", [(1, 1), (3, 1), (1, 3)])
+def test_w8a8_tile_kernel_bands(M, N, split, red):
+    """The banded tile order (past 12 token blocks: bands of 4 channel blocks, the last one narrower) on whole, K-split
+    and 128-token workgroups: 14 and 13 token blocks of 256, 6 and 2 channel blocks, and M = 3072 on the other side of
+    the line (12 of 256, 24 of 128).  Integer sums: bit for bit."""
+    K = 192
+    x, w, s = random_case(M, N, K, M + N)
+    ref = P.w8a8_reference(x, w.t(), s, None, torch.bfloat16)
+    for layout, wp, ldw in ((qf.TILED, qf.to_tiled(w.t()), 0), (qf.ROWMAJOR, w, K)):
+        for x_tiled in (False, True):
+            y = torch.full((M, N + 8), float("nan"), dtype=torch.bfloat16, device=DEV)
+            cfg = (L.KERNEL_MFMA_W8A8_TILE, split, 8, 8, 4, 1, 1, red)
+            w8a8_into(x, wp, s, layout, ldw, y, torch.bfloat16, cfg, x_tiled)
+            assert torch.equal(bits(y[:, :N]), bits(ref)), (layout, x_tiled)
+            assert torch.isnan(y[:, N:].float()).all(), (layout, x_tiled)
+
+
 @pytest.mark.parametrize("M,N,K", [(2048, 8192, 128), (2048, 8000, 128)])
 def test_w8a8_tile_kernel_whole_rounds(M, N, K):
     """Tile grids that are whole rounds of 256 workgroups (rest 0: 32 channel blocks x 8 token blocks) run in

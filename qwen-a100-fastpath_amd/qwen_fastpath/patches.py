@@ -28,7 +28,8 @@ from typing import Callable, NamedTuple, Optional
 import torch
 
 from . import _lib as L
-from .w8a16 import (ROWMAJOR, SMALL_M, TILED, _workspace, from_tiled, pick_config, tiled_numel, to_tiled, w8a16_mm,
+from .w8a16 import _launch as launch_w8a16
+from .w8a16 import (AUTO, ROWMAJOR, SMALL_M, TILED, _workspace, from_tiled, pick_config, tiled_numel, to_tiled, w8a16_mm,
                     w8a16_mm_argmax, w8a16_mm_prefill, w8a8_mm)
 
 logger = logging.getLogger("vllm.qwen_fastpath")
@@ -362,7 +363,9 @@ def _qf_int8_linear_impl(x: torch.Tensor, w_q: torch.Tensor, w_s: torch.Tensor,
         s = w_s.reshape(-1)
         if s.dtype != torch.float32:
             s = s.float()
-        y = w8a16_mm(x2, w_q, s, None, x.dtype, layout)
+        # The body of an op already: w8a16_mm's launch itself, not a second op inside this one (a call at M = 1,
+        # 5120 x 5120 with a bias, 28.8 -> 23.4 us, all of it host time).
+        y = launch_w8a16(x2, w_q, s, layout, x.dtype, AUTO)
         if bias is not None:
             y = y + bias
         return y.view(*lead, N)

@@ -60,6 +60,7 @@ constexpr int kMaxBalanced = kWave;                // requests of a balanced cal
 constexpr size_t kMaxLds = 160 * 1024;             // gfx950 LDS per workgroup
 static_assert(kMaxBalanced * sizeof(int2) <= QF_SPEC_ATTN_PLAN_BYTES, "a slot range a request");
 constexpr int kMaxRows = QF_SPEC_ATTN_MAX_ROWS;
+constexpr int kMaxChunk = 0x7fffffff / kKeyBlock * kKeyBlock;  // the longest split: any larger min_chunk means one split
 constexpr int kNonTemporal = 2;  // cache-policy operand of a direct-to-LDS load: read once
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr size_t kMaxDynLds = 160 * 1024 - 8 * 1024;  // gfx950 LDS per workgroup, less the static arrays
@@ -103,7 +104,8 @@ struct AttnArgs {
 };
 
 // Positions per prefix split (the reference's split arithmetic, spec_attn.py:38-40, with this
-// kernel's key block): both kernels derive it from the sequence length alone.
+// kernel's key block): both kernels derive it from the sequence length alone.  Lengths are below
+// kMaxChunk and run bounds min_chunk by it, so the rounding up stays in range.
 __device__ __forceinline__ int split_chunk(int prefix, const AttnArgs& a) {
   int c = prefix > 0 ? divide(prefix - 1, a.by_splits) + 1 : 0;
   c = c > a.min_chunk ? c : a.min_chunk;
@@ -125,22 +127,24 @@ __device__ __forceinline__ int wave_scan(int v) {
 // chunk length for all requests, the shortest of a rising sequence of multiples of kKeyBlock whose splits fit the
 // a.splits slots of a kv head, so the longest split of a ragged batch is about the batch's mean and not the longest
 // request's share.  A request without a prefix takes one split (its in-flight positions).  Slots go to the requests
-// in order.  Lane i returns request i's length, splits (n) and first slot; `total` slots are used.
+// in order.  Lane i returns request i's length, splits (n) and first slot; `total` slots are used.  In unsigned
+// arithmetic and in units of kKeyBlock, so that min_chunk may be any int and the batch hold up to 2^36 positions.
 __device__ __forceinline__ void balance(const AttnArgs& a, int lane, int& seq, int& chunk, int& n, int& first, int& total) {
   seq = lane < a.B ? a.seq_lens[lane] : 0;
-  const int prefix = max(seq - a.Q, 0);
-  // total positions: at most 64 requests of below 2^31, in units of kKeyBlock so that the sum fits
-  const int units = __builtin_amdgcn_readlane(wave_scan((prefix + kKeyBlock - 1) / kKeyBlock), kWave - 1);
-  const int lo = max((units + a.splits - 1) / a.splits, (a.min_chunk + kKeyBlock - 1) / kKeyBlock);
-  chunk = lo * kKeyBlock;
-  for (;;) {  // ends: once chunk covers the longest prefix, every request takes one split and a.B <= a.splits
-    n = lane < a.B ? max((prefix + chunk - 1) / chunk, 1) : 0;
+  const uint32_t prefix = (uint32_t)max(seq - a.Q, 0);
+  const uint32_t units =
+      (uint32_t)__builtin_amdgcn_readlane(wave_scan((int)((prefix + kKeyBlock - 1) / kKeyBlock)), kWave - 1);
+  const uint32_t lo = max((units + a.splits - 1) / (uint32_t)a.splits, ((uint32_t)a.min_chunk + kKeyBlock - 1) / kKeyBlock);
+  uint32_t len = lo * kKeyBlock;
+  for (;;) {  // ends: once len covers the longest prefix, every request takes one split and a.B <= a.splits
+    n = lane < a.B ? (prefix > 0 ? (int)((prefix - 1) / len) + 1 : 1) : 0;
     const int upto = wave_scan(n);
     first = upto - n;
     total = __builtin_amdgcn_readlane(upto, kWave - 1);
     if (total <= a.splits) break;
-    chunk += (chunk / 8 + kKeyBlock - 1) / kKeyBlock * kKeyBlock;
+    len += (len / 8 + kKeyBlock - 1) / kKeyBlock * kKeyBlock;
   }
+  chunk = (int)min(len, (uint32_t)kMaxChunk);
 }
 
 // s_waitcnt with vmcnt = n (0..63) and the other counters unconstrained.
@@ -334,9 +338,10 @@ spec_prefix_kernel(AttnArgs a) {
   // when the prefix is empty) also takes this step's in-flight positions [prefix, seq).  Query qi sees
   // the positions up to seq - q_len + qi, which include the whole prefix, so one causal bound per
   // row covers both kinds of position.
-  const int start = split * chunk;
-  const bool active = split == 0 || start < prefix;
-  const int end = start + chunk >= prefix ? seq : start + chunk;
+  const int64_t first_pos = (int64_t)split * chunk;  // past 2^31 for the unused splits of a large min_chunk
+  const bool active = split == 0 || first_pos < prefix;
+  const int start = active ? (int)first_pos : 0;
+  const int end = chunk >= prefix - start ? seq : start + chunk;
   if (a.plan != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && wave == 0 && lane < a.B) a.plan[lane] = make_int2(first, n);
   if (!active || start >= end) {
     // no position here: the split's rows get log-sum-exp -inf, so the combine kernel can read every
@@ -839,7 +844,7 @@ int run(const uint16_t* query, int64_t q_stride_tok, int64_t q_stride_head, cons
   a.R = R;
   a.page = page_size;
   a.splits = num_splits;
-  a.min_chunk = min_chunk;
+  a.min_chunk = min_chunk < kMaxChunk ? min_chunk : kMaxChunk;
   a.qk_scale = scale * kLog2e;
   a.by_g = divisor(G);
   a.by_splits = divisor(num_splits);

@@ -84,6 +84,17 @@ def test_split_settings(num_splits, min_chunk):
     _check(inp, _run(inp, num_splits=num_splits, min_chunk=min_chunk), f"splits={num_splits} min_chunk={min_chunk}")
 
 
+@pytest.mark.parametrize("min_chunk", [1 << 26, 1 << 30, (1 << 31) - 40, (1 << 31) - 1])
+@pytest.mark.parametrize("B,num_splits", [(1, None), (3, None), (2, 64), (1, 65535)])
+def test_min_chunk_past_every_length(min_chunk, B, num_splits):
+    """A min_chunk longer than any request means one split each, whatever split * min_chunk comes to: the unused splits
+    take no position and the result is that of num_splits=1, bit for bit."""
+    inp = A.gen_spec_inputs(700, 3, B, H=8, HKV=2, D=64, page=16, seed=B)
+    out = _run(inp, num_splits=num_splits, min_chunk=min_chunk)
+    _check(inp, out, f"min_chunk={min_chunk} B={B} splits={num_splits}")
+    assert np.array_equal(out.view(np.uint32), _run(inp, num_splits=1).view(np.uint32))
+
+
 def test_split_spanning_several_table_windows():
     # one split over 20000 positions of 16-position pages: 1251 pages, more than one 1024-entry window
     inp = A.gen_spec_inputs(20000, 3, 1, H=16, HKV=2, D=128, page=16, seed=77)

@@ -72,7 +72,7 @@ struct GemmArgs {
   int out_f32;
   int vec_out;     // rows of y are 8-byte (bf16) / 16-byte (fp32) aligned: vector stores allowed
   int fused_reduce;  // MFMA, split_k > 1: the last workgroup of an n-block reduces (else a second kernel)
-  // Fused argmax (MFMA, split_k == 1): ids[m] = index_offset + argmax over n < n_valid of the bf16
+  // Fused argmax (split_k == 1): ids[m] = index_offset + argmax over n < n_valid of the bf16
   // outputs y[m, n] (NaN highest, then value, then the lowest index); y may be null.  Each wavefront
   // column folds its candidate per token into one of the token's kArgmaxSlots slots (a 64-bit atomic
   // maximum of argmax_key); argmax_slots_kernel folds the slots into ids and clears them.
@@ -513,11 +513,31 @@ __device__ __forceinline__ void split_range(int split, int splits, int ksteps, i
 // bf16 rounding of an fp32 value, widened back (the value a bf16 output holds)
 __device__ __forceinline__ float bf16_value(float v) { return __uint_as_float((uint32_t)bf16_rne(v) << 16); }
 
-// Fused argmax epilogue of the MFMA kernel (split_k == 1).  Each lane ranks its scaled outputs (bf16
-// values, columns < n_valid) per token, the lanes of a token fold by shuffles, and each wavefront
-// column folds its candidate into the token's slot with one 64-bit atomic maximum of argmax_key (the
-// maximum of keys is the argmax whatever the order of arrival).  The atomics return nothing: no wait,
-// no barrier, the workgroup leaves at once; argmax_slots_kernel reads the slots after the kernel.
+// Fused argmax (split_k == 1), in the epilogue of every kernel that an automatic call without a K split may run, so
+// that the ids are those of the logits it stores.  Each lane ranks its scaled outputs (bf16 values, columns < n_valid)
+// per token, the lanes of a token fold by shuffles, and each wavefront (column) folds its candidate into the token's
+// slot with one 64-bit atomic maximum of argmax_key (the maximum of keys is the argmax whatever the order of arrival).
+// The atomics return nothing: no wait, no barrier, the workgroup leaves at once; argmax_slots_kernel reads the slots
+// after the kernel.
+__device__ __forceinline__ void argmax_fold4(const GemmArgs& a, const f32x4_t v, int n, float& bv, int& bi) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (n + i < a.n_valid) argmax_fold(bf16_value(v[i]), n + i, bv, bi);
+}
+// lanes r, r + 16, r + 32, r + 48 hold token r's candidates
+__device__ __forceinline__ void argmax_slot(const GemmArgs& a, float bv, int bi, int lane, int column, bool writes) {
+#pragma unroll
+  for (int off = 16; off <= 32; off <<= 1) {
+    const float ov = __shfl_xor(bv, off);
+    const int oi = __shfl_xor(bi, off);
+    argmax_fold(ov, oi, bv, bi);
+  }
+  if (writes && lane < a.M)
+    (void)__hip_atomic_fetch_max(a.am_slots + ((int64_t)(column % kArgmaxSlots) * a.M + lane) * argmax_slot_stride(a.M),
+                                 argmax_key(bv, bi), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// ... of the MFMA kernel
 template <int NT, int WN>
 __device__ __forceinline__ void argmax_epilogue(const GemmArgs& a, const f32x4_t (&acc)[NT], bool holder, int tile0,
                                                 int ntiles, int g, int wk, int wn, int lane) {
@@ -538,26 +558,49 @@ __device__ __forceinline__ void argmax_epilogue(const GemmArgs& a, const f32x4_t
     for (int t = 0; t < NT; ++t) {
       const int tile = tile0 + t;
       const int n = tile * kTileN + 4 * g;
-      if (tile < ntiles && n < a.n_valid) {
-        const f32x4_t v = acc[t] * load_scale4(a.scale, a.N, n);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (n + i < a.n_valid) argmax_fold(bf16_value(v[i]), n + i, bv, bi);
-      }
+      if (tile < ntiles && n < a.n_valid) argmax_fold4(a, acc[t] * load_scale4(a.scale, a.N, n), n, bv, bi);
     }
   }
-  // lanes r, r + 16, r + 32, r + 48 hold token r's candidates
+  argmax_slot(a, bv, bi, lane, (int)(blockIdx.x * WN + wn), wk == 0);
+}
+
+// The end of the stream kernels: wavefront v sums the tiles v, v + W, ... of the workgroup's run (tile t0 + t tstep) from
+// the W partial tiles parked in LDS, in wavefront order, and writes them.  Lane (g, r) holds
+// C[n = tile * 16 + 4 g + i][m = r], i = 0..3, in each partial.  The fused argmax has a loop of its own: with one
+// loop for both gate_up at M = 5 took 0.4 us more.  Fused, 32000 x 5120: TILED M = 7 31.1 us (34.5 on the MFMA kernel),
+// row-major M = 4 32.6 (38.0).
+template <int W>
+__device__ __forceinline__ void store_run(const GemmArgs& a, const f32x4_t* part, int t0, int tstep, int nt, int v,
+                                          int lane) {
+  const int g = lane >> 4, r = lane & 15;
+  auto tile_sum = [&](int t) {
+    f32x4_t sum = part[(t * W) * kWave + lane];
 #pragma unroll
-  for (int off = 16; off <= 32; off <<= 1) {
-    const float ov = __shfl_xor(bv, off);
-    const int oi = __shfl_xor(bi, off);
-    argmax_fold(ov, oi, bv, bi);
+    for (int u = 1; u < W; ++u) sum += part[(t * W + u) * kWave + lane];
+    return sum;
+  };
+  if (!a.argmax) {
+    for (int t = v; t < nt; t += W) {
+      const f32x4_t sum = tile_sum(t);
+      const int n = (t0 + t * tstep) * kTileN + 4 * g;
+      if (r < a.M && n < a.N)
+        store_out4(a.y, a.ldy, a.out_f32, a.vec_out, r, n, min(4, a.N - n), sum * load_scale4(a.scale, a.N, n));
+    }
+    return;
   }
-  if (wk == 0 && lane < a.M) {
-    const int slot = (int)((blockIdx.x * WN + wn) % kArgmaxSlots);
-    (void)__hip_atomic_fetch_max(a.am_slots + ((int64_t)slot * a.M + lane) * argmax_slot_stride(a.M),
-                                 argmax_key(bv, bi), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  float bv = -__builtin_inff();
+  int bi = 0x7fffffff;
+#pragma unroll 1
+  for (int t = v; t < nt; t += W) {
+    const f32x4_t sum = tile_sum(t);
+    const int n = (t0 + t * tstep) * kTileN + 4 * g;
+    if (r < a.M && n < a.N) {
+      const f32x4_t y = sum * load_scale4(a.scale, a.N, n);
+      if (a.y != nullptr) store_out4(a.y, a.ldy, a.out_f32, a.vec_out, r, n, min(4, a.N - n), y);
+      argmax_fold4(a, y, n, bv, bi);
+    }
   }
+  argmax_slot(a, bv, bi, lane, (int)blockIdx.x * W + v, true);  // a wavefront without a tile: the least candidate
 }
 
 // Second pass of the fused argmax: one wavefront per token; lane s reads slot s (every atomic maximum of the
@@ -980,15 +1023,7 @@ __global__ void __launch_bounds__(W * kWave) w8a16_stream_kernel(const GemmArgs 
     }
   }
   lds_barrier();
-  // Lane (g, r) holds C[n = tile * 16 + 4 g + i][m = r], i = 0..3, in each partial.
-  for (int t = v; t < nt; t += W) {
-    f32x4_t sum = part[(t * W) * kWave + lane];
-#pragma unroll
-    for (int u = 1; u < W; ++u) sum += part[(t * W + u) * kWave + lane];
-    const int n = (t0 + t * tstep) * kTileN + 4 * g;
-    if (r < a.M && n < a.N)
-      store_out4(a.y, a.ldy, a.out_f32, a.vec_out, r, n, min(4, a.N - n), sum * load_scale4(a.scale, a.N, n));
-  }
+  store_run<W>(a, part, t0, tstep, nt, v, lane);
 }
 
 // The stream kernel with each wavefront's x fragments in registers instead of a staged LDS slice
@@ -1065,14 +1100,7 @@ __global__ void __launch_bounds__(W * kWave) w8a16_stream_xreg_kernel(const Gemm
     acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
   }
   lds_barrier();
-  for (int t = v; t < nt; t += W) {
-    f32x4_t sum = part[(t * W) * kWave + lane];
-#pragma unroll
-    for (int u = 1; u < W; ++u) sum += part[(t * W + u) * kWave + lane];
-    const int n = (t0 + t * tstep) * kTileN + 4 * g;
-    if (r < a.M && n < a.N)
-      store_out4(a.y, a.ldy, a.out_f32, a.vec_out, r, n, min(4, a.N - n), sum * load_scale4(a.scale, a.N, n));
-  }
+  store_run<W>(a, part, t0, tstep, nt, v, lane);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1220,6 +1248,10 @@ __global__ void __launch_bounds__(kRowsWaves * kWave) __attribute__((amdgpu_wave
     for (int t = 0; t < nt; ++t) part[(t * W + v) * kWave + lane] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
   }
   __syncthreads();
+  if (a.split_k == 1) {
+    store_run<W>(a, part, t0, 1, nt, v, lane);
+    return;
+  }
   // Lane (g, r) holds C[n = tile * 16 + 4 g + i][m = r], i = 0..3, in each partial.
   const int64_t plane = (int64_t)a.M * a.n_pad;
   for (int t = v; t < nt; t += W) {
@@ -1227,16 +1259,12 @@ __global__ void __launch_bounds__(kRowsWaves * kWave) __attribute__((amdgpu_wave
 #pragma unroll
     for (int u = 1; u < W; ++u) sum += part[(t * W + u) * kWave + lane];
     const int n = (t0 + t) * kTileN + 4 * g;
-    if (a.split_k == 1) {
-      if (r < a.M && n < a.N)
-        store_out4(a.y, a.ldy, a.out_f32, a.vec_out, r, n, min(4, a.N - n), sum * load_scale4(a.scale, a.N, n));
-    } else if (r < a.M) {
+    if (r < a.M) {
       float* dst = a.partial + (int64_t)blockIdx.y * plane + (int64_t)r * a.n_pad + n;
 #pragma unroll
       for (int i = 0; i < 4; ++i) __hip_atomic_store(dst + i, sum[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
-  if (a.split_k == 1) return;
   // Last arrival, ordered as in w8a16_mfma_kernel.
   __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
   __syncthreads();
@@ -3325,7 +3353,7 @@ bool auto_config(int M, int N, int K, int layout, qf_w8a16_config* c, bool strea
 }
 
 // Validate / complete a caller configuration.
-// stream_ok = false for the fused argmax, whose epilogue only the MFMA kernels have.
+// stream_ok = false for the question whether the fused argmax is served (argmax_served).
 int resolve_config(int M, int N, int K, int layout, const qf_w8a16_config* in, qf_w8a16_config* out,
                    bool stream_ok = true) {
   if (!auto_config(M, N, K, layout, out, stream_ok)) return QF_ERR_UNSUPPORTED;
@@ -3375,7 +3403,7 @@ struct RowsPlan {
 
 // The least time of the busiest wavefront, in pairs (tiles of a run times pairs a tile), over the splits up to max_split
 // (the planes that the caller's workspace holds) that run in one round of workgroups, one a CU, with a run's partial
-// tiles in LDS (15 tiles: up to 61440 channels; a vocabulary keeps the MFMA kernel, whose sums its fused argmax shares);
+// tiles in LDS (15 tiles: up to 61440 channels; a larger vocabulary keeps the MFMA kernel);
 // a split costs about a pair and a half, its partials' round trip: qkv 10240 x 5120
 // at M = 5 3 x 5 unsplit 13.1 us, 5 x 3 in two splits 14.8; o_proj 5120 x 8192 2 x 8 unsplit 13.8, 3 x 4 in two 13.6.
 RowsPlan rows_plan(int N, int K, int max_split) {
@@ -3420,6 +3448,9 @@ struct ArgmaxRequest {
   int64_t* ids;
 };
 
+// The fused argmax is served where the MFMA kernel would run without a K split.
+bool argmax_served(const qf_w8a16_config& c) { return is_mfma(c.kernel) && c.split_k == 1; }
+
 // Workspace of the fused argmax: the counter prefix, which holds the per-token slots.
 size_t argmax_workspace_for(const qf_w8a16_config&, int, int) { return QF_W8A16_COUNTER_BYTES; }
 
@@ -3437,9 +3468,14 @@ int run_gemm(const uint16_t* x, int64_t ldx, const int8_t* w, int64_t ldw, int l
   if (ldx % 8 || (layout == QF_LAYOUT_ROWMAJOR && ldw % 16)) return QF_ERR_UNSUPPORTED;
 
   qf_w8a16_config c;
-  const int rc = resolve_config(M, N, K, layout, cfg, &c, am == nullptr);
+  int rc = resolve_config(M, N, K, layout, cfg, &c, am == nullptr);
   if (rc != QF_OK) return rc;
-  if (am != nullptr && (!is_mfma(c.kernel) || c.split_k != 1)) return QF_ERR_UNSUPPORTED;
+  const bool automatic = cfg == nullptr || cfg->kernel == QF_KERNEL_AUTO;
+  if (am != nullptr) {
+    if (!argmax_served(c)) return QF_ERR_UNSUPPORTED;
+    // the kernel of the plain call, so that the ids are those of its logits
+    if (automatic && (rc = resolve_config(M, N, K, layout, cfg, &c)) != QF_OK) return rc;
+  }
   // The normalising GEMM needs whole rows staged: no K split, and an instantiation that normalises.
   if (norm_eps != nullptr && (c.split_k != 1 || select_norm(c, layout) == nullptr)) return QF_ERR_UNSUPPORTED;
   const size_t need = am != nullptr ? argmax_workspace_for(c, M, N) : workspace_for(c, M, N);
@@ -3480,22 +3516,13 @@ int run_gemm(const uint16_t* x, int64_t ldx, const int8_t* w, int64_t ldw, int l
 
   const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   // Row-major weights at 2 or more tokens, automatic calls: whole-line copies (M = 1: the GEMV's row reads stay ahead on
-  // narrow N, qkv 11.9 against 12.6 us; the fused argmax and the normalising GEMM are epilogues of the other kernels).
-  if (layout == QF_LAYOUT_ROWMAJOR && M >= 2 && am == nullptr && norm_eps == nullptr &&
-      (cfg == nullptr || cfg->kernel == QF_KERNEL_AUTO)) {
-    const RowsPlan p = rows_plan(N, K, c.split_k);
-    if (p.columns > 0) {
-      a.split_k = p.split;
-      a.counter_stride = counter_stride_for(p.columns);
-      const bool lines = ldw % 128 == 0 && (reinterpret_cast<uintptr_t>(w) & 127) == 0;
-      return launch(lines ? rows_by_pairs<true>(p.pairs) : rows_by_pairs<false>(p.pairs), dim3(p.columns, p.split), dim3(kRowsWaves * kWave),
-                    (size_t)kRowsRing + (size_t)p.run * kRowsWaves * kWave * sizeof(f32x4_t), s, a);
-    }
-  }
-  const dim3 grid = c.kernel == QF_KERNEL_MFMA_WIDE ? dim3(workgroups(c, N) * a.groups * c.split_k)
-                                                    : dim3(workgroups(c, N), c.split_k);
-  const dim3 block(c.waves * kWave);
-  const size_t smem = lds_bytes(c, M, a.ksteps, N);
+  // narrow N, qkv 11.9 against 12.6 us; the normalising GEMM is an epilogue of the other kernels).
+  RowsPlan rows{0, 0, 0, 0};
+  if (layout == QF_LAYOUT_ROWMAJOR && M >= 2 && norm_eps == nullptr && automatic) rows = rows_plan(N, K, c.split_k);
+  dim3 grid = c.kernel == QF_KERNEL_MFMA_WIDE ? dim3(workgroups(c, N) * a.groups * c.split_k)
+                                              : dim3(workgroups(c, N), c.split_k);
+  dim3 block(c.waves * kWave);
+  size_t smem = lds_bytes(c, M, a.ksteps, N);
   KernelFn fn = (c.kernel == QF_KERNEL_GEMV)
                     ? select_gemv(M, c.tiles_per_wave, c.waves, c.load_hint)
                 : (c.kernel == QF_KERNEL_MFMA_STREAM)
@@ -3506,6 +3533,16 @@ int run_gemm(const uint16_t* x, int64_t ldx, const int8_t* w, int64_t ldw, int l
                     : select_mfma(layout, c.tiles_per_wave, c.waves, c.k_waves, c.depth, c.load_hint,
                                   c.kernel == QF_KERNEL_MFMA_XRING);
   if (norm_eps != nullptr) fn = select_norm(c, layout);
+  if (rows.columns > 0) {
+    a.split_k = rows.split;
+    a.fused_reduce = 1;
+    a.counter_stride = counter_stride_for(rows.columns);
+    const bool lines = ldw % 128 == 0 && (reinterpret_cast<uintptr_t>(w) & 127) == 0;
+    fn = lines ? rows_by_pairs<true>(rows.pairs) : rows_by_pairs<false>(rows.pairs);
+    grid = dim3(rows.columns, rows.split);
+    block = dim3(kRowsWaves * kWave);
+    smem = (size_t)kRowsRing + (size_t)rows.run * kRowsWaves * kWave * sizeof(f32x4_t);
+  }
   if (fn == nullptr) return QF_ERR_UNSUPPORTED;
   int st = launch(fn, grid, block, smem, s, a);
   if (st != QF_OK) return st;
@@ -4041,8 +4078,7 @@ int qf_w8a16_gemm_noalloc(const uint16_t* x, int64_t ldx, const int8_t* w, int64
 
 size_t qf_w8a16_argmax_workspace_bytes(int M, int N, int K, int layout, const qf_w8a16_config* cfg) {
   qf_w8a16_config c;
-  if (resolve_config(M, N, K, layout, cfg, &c, false) != QF_OK) return 0;
-  if (!is_mfma(c.kernel) || c.split_k != 1) return 0;
+  if (resolve_config(M, N, K, layout, cfg, &c, false) != QF_OK || !argmax_served(c)) return 0;
   return argmax_workspace_for(c, M, N);
 }
 

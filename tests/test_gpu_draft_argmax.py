@@ -64,6 +64,29 @@ def test_fused_ids_equal_unfused(oracle, layout, M, N, K):
         assert np.array_equal(ids_only.cpu().numpy(), ref)
 
 
+@pytest.mark.parametrize("layout", [qf.TILED, qf.ROWMAJOR])
+@pytest.mark.parametrize("N,K", [(32000, 5120), (50257, 1024), (16399, 4096), (61441, 2112), (12000, 576)])
+def test_fused_kernel_is_the_plain_one(layout, N, K):
+    """Vocabularies that the plain call gives to the stream kernels: the fused call stores the same logits bit for bit
+    and its ids are their argmax, with near ties (every logit of a row within a few bf16 steps of another's)."""
+    w, s = _head(N, K, seed=N, plant=False)
+    wl = qf.to_tiled(w.t()) if layout == qf.TILED else w.t()
+    served = []
+    for M in (2, 3, 4, 5, 7, 8, 12, 16):
+        g = torch.Generator(device=DEV)
+        g.manual_seed(M)
+        x = torch.randn(M, K, device=DEV, generator=g).to(torch.bfloat16)
+        res = qf.w8a16_mm_argmax(x, wl, s, N - 3, 9, None, layout, with_logits=True)
+        if res is None:
+            continue
+        served.append(M)
+        y = qf.w8a16_mm(x, wl, s, None, torch.bfloat16, layout)
+        assert torch.equal(res[1].view(torch.int16), y.view(torch.int16)), M
+        assert torch.equal(res[0], qf.top_tokens(y, 3, 9)), M
+        assert torch.equal(qf.w8a16_mm_argmax(x, wl, s, N - 3, 9, None, layout), res[0]), M
+    assert {4, 5, 7} <= set(served), served
+
+
 def test_nan_row_and_all_pad_winner(oracle):
     N, K, M = 3000, 512, 3
     w, s = _head(N, K, seed=5, plant=False)

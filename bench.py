@@ -55,6 +55,14 @@ PROFILE_SUMMARY = os.path.join(ROOT, "profiles", "w8a16_layer_m5_pmc.md")
 W8A8_PROFILE = os.path.join(ROOT, "profiles", "w8a8_gate_up_m2048_pmc.txt")
 
 
+def launch_config(qf, M: int, N: int, K: int, layout: int) -> dict:
+    """What an automatic call launches: the row stream kernel's plan on row-major weights where it serves the call
+    (runs, tiles a run, K splits, pairs a wavefront), else the resolved configuration."""
+    from qwen_fastpath import _lib as QL
+    plan = QL.rows_plan(M, N, K) if layout == qf.ROWMAJOR else None
+    return {"rows_plan": list(plan)} if plan else {"config": list(qf.resolve_config(M, N, K, layout))}
+
+
 def algo_bytes(M: int, N: int, K: int) -> int:
     """Compulsory bytes: int8 weights + fp32 scales + bf16 activations + bf16 outputs."""
     return N * K + 4 * N + 2 * M * K + 2 * M * N
@@ -277,7 +285,7 @@ def main():
             sets[i % len(sets)].gemm(qf, torch, args.profile_gemm, cfg)
         torch.cuda.synchronize()
         log(f"profile: {args.iters} launches of {args.profile_gemm} M={M_TOKENS} N={N} K={K} layout={args.layout} "
-            f"cfg={tuple(cfg) if cfg else tuple(qf.resolve_config(M_TOKENS, N, K, layout))}")
+            f"{'cfg=' + str(tuple(cfg)) if cfg else launch_config(qf, M_TOKENS, N, K, layout)}")
         return
 
     if args.workload == "stack64":
@@ -361,13 +369,13 @@ def main():
             times.append(e0.elapsed_time(e1) * 1e3 / launches)
         us = sorted(times)[len(times) // 2]
         b = algo_bytes(M, N, K)
-        cfg = qf.resolve_config(M, N, K, layout)
+        cfg = launch_config(qf, M, N, K, layout)
         per_gemm[name] = {"N": N, "K": K, "us": round(us, 2), "best_us": round(min(times), 2),
                           "weight_sets_rotated": len(sets), "rotated_MB": round(len(sets) * N * K / 1e6, 1),
                           "GB_s": round(b / us / 1e3, 1), "weight_GB_s": round(N * K / us / 1e3, 1),
-                          "pct_peak": round(100 * b / us / 1e3 / PEAK_GBS, 1), "config": list(cfg)}
+                          "pct_peak": round(100 * b / us / 1e3 / PEAK_GBS, 1), **cfg}
         log(f"  {name:8s} N={N:6d} K={K:6d}: {us:7.2f} us  {b / us / 1e3:7.0f} GB/s  "
-            f"{100 * b / us / 1e3 / PEAK_GBS:5.1f}%  cfg={tuple(cfg)}")
+            f"{100 * b / us / 1e3 / PEAK_GBS:5.1f}%  {cfg}")
         if name == DOMINANT:
             dominant_us = us
         del g, sets
@@ -390,7 +398,7 @@ def main():
     b1 = algo_bytes(1, N1, K1)
     single = {"N": N1, "K": K1, "M": 1, "us": round(us1, 2), "best_us": round(best1[0], 2),
               "GB_s": round(b1 / us1 / 1e3, 1), "weight_GB_s": round(N1 * K1 / us1 / 1e3, 1),
-              "pct_peak": round(100 * b1 / us1 / 1e3 / PEAK_GBS, 1), "config": list(qf.resolve_config(1, N1, K1, layout))}
+              "pct_peak": round(100 * b1 / us1 / 1e3 / PEAK_GBS, 1), **launch_config(qf, 1, N1, K1, layout)}
     log(f"  single linear M=1 N=K=5120: {us1:7.2f} us  {b1 / us1 / 1e3:7.0f} GB/s  {100 * b1 / us1 / 1e3 / PEAK_GBS:5.1f}%")
     del sets1
     release_cache(torch)
@@ -581,7 +589,7 @@ def msweep_rows(torch, qf, dev, layout, layers=None) -> dict:
                                         for _ in range(reps) for i, (w, s) in enumerate(sets)], reps * R)
         b = algo_bytes(M, N, K)
         rows[M] = {"us": round(us, 2), "GB_s": round(b / us / 1e3, 1), "pct_peak": round(100 * b / us / 1e3 / PEAK_GBS, 1),
-                   "config": list(qf.resolve_config(M, N, K, layout))}
+                   **launch_config(qf, M, N, K, layout)}
         log(f"  gate_up M={M:2d}: {us:7.2f} us  {b / us / 1e3:7.0f} GB/s  {100 * b / us / 1e3 / PEAK_GBS:5.1f}%")
     del sets
     torch.cuda.empty_cache()
@@ -843,7 +851,7 @@ def run_tp8(torch, qf, dev, args):
         b = algo_bytes(M, N, K)
         rows[name] = {"N": N, "K": K, "us": round(us, 2), "GB_s": round(b / us / 1e3, 1),
                       "pct_peak": round(100 * b / us / 1e3 / PEAK_GBS, 1),
-                      "config": list(qf.resolve_config(M, N, K, layout))}
+                      **launch_config(qf, M, N, K, layout)}
         log(f"  tp8 {name:8s} N={N:5d} K={K:5d}: {us:6.2f} us  {b / us / 1e3:6.0f} GB/s  {100 * b / us / 1e3 / PEAK_GBS:5.1f}%")
     us_layer = time_graph(torch, lambda: [gemm(L_, n) for _ in range(4) for L_ in layers for n in TP8_GEMMS], 4 * R)
     b_layer = sum(algo_bytes(M, N, K) for N, K in TP8_GEMMS.values())

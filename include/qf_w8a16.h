@@ -125,14 +125,20 @@ int qf_abi_version(void);
 /* Static text for a qf_status value. */
 const char* qf_status_string(int status);
 
-/* Fill *cfg with the configuration used for (M, N, K, layout).  Returns QF_ERR_UNSUPPORTED when the
+/* Fill *cfg with the automatic configuration for (M, N, K, layout).  Returns QF_ERR_UNSUPPORTED when the
  * shape is not served (M < 1, M > 16 on row-major weights, N < 1, K % 64 != 0, unknown layout),
  * mirroring pick_config() returning None.  M > 16 on TILED weights gets QF_KERNEL_MFMA_WIDE (the
  * reference sends M > 16 to its W8A8 fallback, plugin/qwen_fastpath/patches.py:99-100, which cannot
  * read the TILED image).  On row-major weights at 2 <= M <= 16 an automatic qf_w8a16_gemm may run the
  * library's row stream kernel instead, which has no explicit form, within this configuration's
- * workspace (its sums differ in order only).  Host-only; touches no device. */
+ * workspace (its sums differ in order only): qf_w8a16_rows_plan says where.  Host-only; touches no device. */
 int qf_w8a16_pick_config(int M, int N, int K, int layout, qf_w8a16_config* cfg);
+
+/* The row stream kernel's launch for an automatic qf_w8a16_gemm or qf_w8a16_gemm_argmax on row-major weights
+ * (128-byte aligned) of row stride ldw: out = {runs of 16-channel tiles, tiles of the longest run, K splits,
+ * pairs of 64-k steps of the busiest wavefront}; runs x K splits workgroups of 8 wavefronts.
+ * QF_ERR_UNSUPPORTED where the call runs qf_w8a16_pick_config's kernel (or is not served).  Host-only. */
+int qf_w8a16_rows_plan(int M, int N, int K, int64_t ldw, int32_t* out);
 
 /* Bytes of device workspace qf_w8a16_gemm needs for this call (0 when split_k == 1): arrival
  * counters followed by the split partial sums.  cfg may be NULL (automatic configuration).

@@ -3432,6 +3432,12 @@ RowsPlan rows_plan(int N, int K, int max_split) {
   return best;
 }
 
+// The row stream kernel's plan for an automatic row-major call (configuration c), columns 0 where c's kernel runs.
+// M = 1: the GEMV's row reads stay ahead on narrow N (qkv 11.9 against 12.6 us).
+RowsPlan rows_for_call(int M, int N, int K, const qf_w8a16_config& c) {
+  return M >= 2 ? rows_plan(N, K, c.split_k) : RowsPlan{0, 0, 0, 0};
+}
+
 // Words between the arrival counters of n workgroup groups: spread over the counter prefix (up to 1 KiB apart),
 // since atomics on nearby addresses share a memory channel (measured on the fused argmax: 64 slots 64 bytes apart
 // cost 11 us on 9496 workgroups, 1 KiB apart about 3).
@@ -3515,10 +3521,9 @@ int run_gemm(const uint16_t* x, int64_t ldx, const int8_t* w, int64_t ldw, int l
   if (c.kernel == QF_KERNEL_MFMA_WIDE) wide_groups(M, a.groups, a.group_rows);
 
   const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  // Row-major weights at 2 or more tokens, automatic calls: whole-line copies (M = 1: the GEMV's row reads stay ahead on
-  // narrow N, qkv 11.9 against 12.6 us; the normalising GEMM is an epilogue of the other kernels).
+  // Row-major weights, automatic calls: whole-line copies (the normalising GEMM is an epilogue of the other kernels).
   RowsPlan rows{0, 0, 0, 0};
-  if (layout == QF_LAYOUT_ROWMAJOR && M >= 2 && norm_eps == nullptr && automatic) rows = rows_plan(N, K, c.split_k);
+  if (layout == QF_LAYOUT_ROWMAJOR && norm_eps == nullptr && automatic) rows = rows_for_call(M, N, K, c);
   dim3 grid = c.kernel == QF_KERNEL_MFMA_WIDE ? dim3(workgroups(c, N) * a.groups * c.split_k)
                                               : dim3(workgroups(c, N), c.split_k);
   dim3 block(c.waves * kWave);
@@ -4033,6 +4038,19 @@ const char* qf_status_string(int status) {
 int qf_w8a16_pick_config(int M, int N, int K, int layout, qf_w8a16_config* cfg) {
   if (cfg == nullptr) return QF_ERR_INVALID_ARG;
   return auto_config(M, N, K, layout, cfg) ? QF_OK : QF_ERR_UNSUPPORTED;
+}
+
+int qf_w8a16_rows_plan(int M, int N, int K, int64_t ldw, int32_t* out) {
+  if (out == nullptr || M < 1 || N < 1 || K < 1 || ldw < K) return QF_ERR_INVALID_ARG;
+  qf_w8a16_config c;
+  if (M > QF_W8A16_MAX_M || ldw % 16 || !auto_config(M, N, K, QF_LAYOUT_ROWMAJOR, &c)) return QF_ERR_UNSUPPORTED;
+  const RowsPlan p = rows_for_call(M, N, K, c);
+  if (p.columns == 0) return QF_ERR_UNSUPPORTED;
+  out[0] = p.columns;
+  out[1] = p.run;
+  out[2] = p.split;
+  out[3] = p.pairs;
+  return QF_OK;
 }
 
 size_t qf_w8a16_workspace_bytes(int M, int N, int K, int layout, const qf_w8a16_config* cfg) {

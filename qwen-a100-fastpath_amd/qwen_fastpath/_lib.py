@@ -43,6 +43,7 @@ EXPORTS = (
     "qf_abi_version",
     "qf_status_string",
     "qf_w8a16_pick_config",
+    "qf_w8a16_rows_plan",
     "qf_w8a16_workspace_bytes",
     "qf_w8a16_gemm",
     "qf_w8a16_gemm_noalloc",
@@ -131,6 +132,8 @@ def load() -> ctypes.CDLL:
     L.qf_status_string.restype = ctypes.c_char_p
     L.qf_w8a16_pick_config.argtypes = [i32, i32, i32, i32, ctypes.POINTER(Config)]
     L.qf_w8a16_pick_config.restype = i32
+    L.qf_w8a16_rows_plan.argtypes = [i32, i32, i32, i64, ctypes.POINTER(ctypes.c_int32)]
+    L.qf_w8a16_rows_plan.restype = i32
     L.qf_w8a16_workspace_bytes.argtypes = [i32, i32, i32, i32, ctypes.POINTER(Config)]
     L.qf_w8a16_workspace_bytes.restype = sz
     L.qf_w8a16_gemm.argtypes = [p, i64, p, i64, i32, p, p, i64, i32, i32, i32, i32,
@@ -230,6 +233,17 @@ def w8a8_pick_config(M: int, N: int, K: int, layout: int = LAYOUT_TILED) -> Conf
         return None
     check(rc, "qf_w8a8_pick_config")
     return c
+
+
+def rows_plan(M: int, N: int, K: int, ldw: int | None = None) -> tuple[int, int, int, int] | None:
+    """The row stream kernel's launch for an automatic call on row-major weights of row stride ldw (K by default): (runs,
+    tiles of the longest run, K splits, pairs of k-steps of the busiest wavefront); None where pick_config's kernel runs."""
+    out = (ctypes.c_int32 * 4)()
+    rc = load().qf_w8a16_rows_plan(M, N, K, K if ldw is None else ldw, out)
+    if rc == ERR_UNSUPPORTED:
+        return None
+    check(rc, "qf_w8a16_rows_plan")
+    return tuple(out)
 
 
 W8A8_LAUNCH_KINDS = ("tile", "tile_256x128", "tile_128x128", "wide", "split_reduce")

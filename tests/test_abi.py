@@ -112,6 +112,35 @@ def test_stream_kernel_rule_host_only():
                      cfg=L.Config.from_seq(bad)) == L.ERR_UNSUPPORTED, bad
 
 
+def test_rows_plan_host_only():
+    """Where an automatic call on row-major weights runs the row stream kernel: every tile in a run, every pair of k-steps
+    at a wavefront, a run's partial tiles in LDS, K splits within the workspace of the reported configuration; the
+    full-width layer's four linears and the tensor-parallel shards among them; not at M = 1, past 61440 channels, on a row
+    stride the kernels do not take."""
+    cus = 256  # no device here
+    for M in (2, 3, 5, 8, 11, 12, 16):
+        for N, K in ((10240, 5120), (5120, 8192), (34816, 5120), (5120, 17408), (1280, 5120), (5120, 1024), (4352, 5120),
+                     (5120, 2176), (1, 64), (17, 192), (61440, 1024), (256, 10304), (12300, 320), (6000, 2112)):
+            plan = L.rows_plan(M, N, K)
+            cfg = L.pick_config(M, N, K, L.LAYOUT_ROWMAJOR)
+            if K % 128 == 0:
+                assert plan is not None, (M, N, K)
+            if plan is None:
+                continue
+            runs, run, split, pairs = plan
+            tiles, all_pairs = (N + 15) // 16, (K // 64 + 1) // 2
+            assert 1 <= runs <= tiles <= runs * run, (M, N, K, plan)
+            assert 1 <= split <= cfg.split_k and runs * split <= cus, (M, N, K, plan)
+            assert pairs <= 10 and 8 * pairs * split >= all_pairs, (M, N, K, plan)
+            assert 32 * 1024 + run * 8 * 1024 <= 160 * 1024 - 256, (M, N, K, plan)
+    assert L.rows_plan(1, 5120, 8192) is None and L.rows_plan(5, 61441, 1024) is None
+    assert L.rows_plan(17, 5120, 8192) is None and L.rows_plan(5, 5120, 8192, 8200) is None
+    assert L.rows_plan(5, 5120, 8192, 8192 + 128) == L.rows_plan(5, 5120, 8192)
+    out = (ctypes.c_int32 * 4)()
+    assert L.load().qf_w8a16_rows_plan(5, 100, 1024, 1000, out) == L.ERR_INVALID_ARG
+    assert L.load().qf_w8a16_rows_plan(5, 100, 1024, 1024, None) == L.ERR_INVALID_ARG
+
+
 def test_workspace_for_explicit_config():
     c = L.Config.from_seq((2, 4, 2, 4, 4, 0, 1))      # 63 tiles / (4 x 2) -> 8 workgroups
     assert L.workspace_bytes(5, 1000, 1024, 0, c) == 65536 + 4 * 5 * 1008 * 4

@@ -3432,10 +3432,37 @@ RowsPlan rows_plan(int N, int K, int max_split) {
   return best;
 }
 
+// Rows that start inside a 128-byte line (K an odd number of steps, or a row stride that is no multiple of 128): the
+// lines at the pairs' ends are fetched by two wavefronts each, and the row kernel can lose to the kernel c that it stands
+// in for where c's grid happens to fill the CUs.  c stays where it does not split K, fills 0.6 of its rounds and does so
+// better than the row plan (1.1 times; 0.9 at M = 2, where c has the least x to stage), and, past 32 steps, where it
+// splits K, fills more than 0.72 of at most two rounds and the row plan walks many tiles a workgroup (30481 x 1088 at
+// M = 4 9.7 us against 11.2; 6341 x 14912 at M = 15 24.6 against 29.9).  Both kernels in turn, 512 to 40000 channels,
+// K 512 to 18500, M 2 to 16: over 1882 calls the row kernel everywhere takes 0.757 of c's time (geometric mean), at worst
+// 1.21; with this rule 0.754 and 1.08; over 1685 further calls 0.765 and 1.26 (88 past 1.03) against 0.755 and 1.14 (14).
+// With whole lines it takes 0.68 over 3800 calls, at worst 1.06, and always runs.
+bool rows_lose_lines(int M, int N, int K, const qf_w8a16_config& c, const RowsPlan& p) {
+  if (c.kernel != QF_KERNEL_MFMA || round_up16(N) / (kTileN * 16) >= 128) return false;  // wide N: at worst 0.90
+  const int ntiles = round_up16(N) / kTileN;
+  const int ksteps = K / kStepK;
+  const int cus = device_cus();
+  const int64_t wgs = (int64_t)workgroups(c, N) * c.split_k;
+  const int64_t rounds = (wgs + cus - 1) / cus;
+  const double fill = (double)wgs / (double)(rounds * cus);
+  if (c.split_k == 1) {
+    const double share = (double)ntiles * ((ksteps + 1) / 2) / ((double)p.run * p.pairs * kRowsWaves * cus);
+    return fill > 0.6 && fill > (M == 2 ? 0.9 : 1.1) * share;
+  }
+  return ksteps > 32 && fill > 0.72 && ((rounds == 1 && p.run >= 3) || (rounds == 2 && p.run >= 8));
+}
+
 // The row stream kernel's plan for an automatic row-major call (configuration c), columns 0 where c's kernel runs.
 // M = 1: the GEMV's row reads stay ahead on narrow N (qkv 11.9 against 12.6 us).
-RowsPlan rows_for_call(int M, int N, int K, const qf_w8a16_config& c) {
-  return M >= 2 ? rows_plan(N, K, c.split_k) : RowsPlan{0, 0, 0, 0};
+RowsPlan rows_for_call(int M, int N, int K, bool lines, const qf_w8a16_config& c) {
+  RowsPlan none{0, 0, 0, 0};
+  if (M < 2) return none;
+  const RowsPlan p = rows_plan(N, K, c.split_k);
+  return p.columns > 0 && !lines && rows_lose_lines(M, N, K, c, p) ? none : p;
 }
 
 // Words between the arrival counters of n workgroup groups: spread over the counter prefix (up to 1 KiB apart),
@@ -3522,8 +3549,9 @@ int run_gemm(const uint16_t* x, int64_t ldx, const int8_t* w, int64_t ldw, int l
 
   const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   // Row-major weights, automatic calls: whole-line copies (the normalising GEMM is an epilogue of the other kernels).
+  const bool lines = ldw % 128 == 0 && (reinterpret_cast<uintptr_t>(w) & 127) == 0;
   RowsPlan rows{0, 0, 0, 0};
-  if (layout == QF_LAYOUT_ROWMAJOR && norm_eps == nullptr && automatic) rows = rows_for_call(M, N, K, c);
+  if (layout == QF_LAYOUT_ROWMAJOR && norm_eps == nullptr && automatic) rows = rows_for_call(M, N, K, lines, c);
   dim3 grid = c.kernel == QF_KERNEL_MFMA_WIDE ? dim3(workgroups(c, N) * a.groups * c.split_k)
                                               : dim3(workgroups(c, N), c.split_k);
   dim3 block(c.waves * kWave);
@@ -3542,7 +3570,6 @@ int run_gemm(const uint16_t* x, int64_t ldx, const int8_t* w, int64_t ldw, int l
     a.split_k = rows.split;
     a.fused_reduce = 1;
     a.counter_stride = counter_stride_for(rows.columns);
-    const bool lines = ldw % 128 == 0 && (reinterpret_cast<uintptr_t>(w) & 127) == 0;
     fn = lines ? rows_by_pairs<true>(rows.pairs) : rows_by_pairs<false>(rows.pairs);
     grid = dim3(rows.columns, rows.split);
     block = dim3(kRowsWaves * kWave);
@@ -4044,7 +4071,7 @@ int qf_w8a16_rows_plan(int M, int N, int K, int64_t ldw, int32_t* out) {
   if (out == nullptr || M < 1 || N < 1 || K < 1 || ldw < K) return QF_ERR_INVALID_ARG;
   qf_w8a16_config c;
   if (M > QF_W8A16_MAX_M || ldw % 16 || !auto_config(M, N, K, QF_LAYOUT_ROWMAJOR, &c)) return QF_ERR_UNSUPPORTED;
-  const RowsPlan p = rows_for_call(M, N, K, c);
+  const RowsPlan p = rows_for_call(M, N, K, ldw % 128 == 0, c);
   if (p.columns == 0) return QF_ERR_UNSUPPORTED;
   out[0] = p.columns;
   out[1] = p.run;

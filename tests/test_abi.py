@@ -136,6 +136,10 @@ def test_rows_plan_host_only():
     assert L.rows_plan(1, 5120, 8192) is None and L.rows_plan(5, 61441, 1024) is None
     assert L.rows_plan(17, 5120, 8192) is None and L.rows_plan(5, 5120, 8192, 8200) is None
     assert L.rows_plan(5, 5120, 8192, 8192 + 128) == L.rows_plan(5, 5120, 8192)
+    # rows that start inside a 128-byte line: the MFMA kernel stays where its grid fills the machine
+    for M, N, K in ((4, 30481, 1088), (2, 13945, 4160), (5, 5000, 2112), (15, 6341, 14912), (16, 9000, 3136)):
+        assert L.rows_plan(M, N, K) is None, (M, N, K)
+        assert L.rows_plan(M, N, K, K + 64) is not None, (M, N, K)  # a row stride of whole lines
     out = (ctypes.c_int32 * 4)()
     assert L.load().qf_w8a16_rows_plan(5, 100, 1024, 1000, out) == L.ERR_INVALID_ARG
     assert L.load().qf_w8a16_rows_plan(5, 100, 1024, 1024, None) == L.ERR_INVALID_ARG

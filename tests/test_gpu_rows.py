@@ -7,6 +7,7 @@ import pytest
 import torch
 
 import qwen_fastpath as qf
+from qwen_fastpath import _lib as L
 from helpers import bf16_bits, dev_inputs
 
 pytestmark = pytest.mark.gpu
@@ -26,6 +27,20 @@ def test_row_stream_shapes(oracle, N, K):
             assert rep.ok, (M, N, K, rep)
         y32 = qf.w8a16_mm(x, w, s, None, torch.float32).cpu()
         assert np.array_equal(bf16_bits(y32.to(torch.bfloat16)), y), (M, N, K)  # the same sums before the rounding
+
+
+@pytest.mark.parametrize("N,K,Ms", [(333, 1984, (2, 16)), (700, 10304, (5, 16)), (9000, 1472, (3, 12)), (9000, 3136, (5,)),
+                                    (12300, 320, (11,)), (40000, 320, (2, 16)), (6000, 2112, (7,))])
+def test_row_stream_half_lines(oracle, N, K, Ms):
+    """Rows that start in the middle of a cache line, on the shapes that the row stream kernel keeps (rows_plan): one
+    tile and up to ten a run, one pair and several, with and without a K split."""
+    for M in Ms:
+        assert L.rows_plan(M, N, K) is not None, (M, N, K)
+        inp = oracle.gen_inputs(M, N, K, seed=M + N + K)
+        x, w, s = dev_inputs(inp, DEV)
+        for _ in range(2):
+            rep = oracle.check_w8a16(bf16_bits(qf.w8a16_mm(x, w, s, None, torch.bfloat16)), inp.x, inp.w, inp.s)
+            assert rep.ok, (M, N, K, rep)
 
 
 def test_row_stream_strided_weights(oracle):

@@ -257,10 +257,12 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
 // Geometry of the prefix kernel for head size D and RT row tiles.
 template <int D, int RT>
 struct Geo {
-  // A stage is one 16-position key tile a wavefront.  4 wavefronts at D = 256 (two stages of 64 positions fill 128 KiB
-  // of LDS) and where 4 row tiles at D = 128 leave no room beside the rings; 8 otherwise, so that two wavefronts share
-  // a SIMD.
-  static constexpr int kWaves = D == 256 || (D == 128 && RT == 4) ? 4 : 8;
+  // A stage is one 16-position key tile a wavefront.  4 wavefronts at D = 256, where two stages of 64 positions fill
+  // 128 KiB of LDS, and at D = 128, where LDS then holds two workgroups a CU, for grids of more workgroups than CUs (8
+  // wavefronts up to 48 rows, 105 to 25000 positions, 1 to 64 requests: 1.08 times the time up to 500 positions, 1.03 to
+  // 2000, 1.00 above).  8 at D = 64: 4 have too few bytes in flight for long contexts (above 2000 positions up to 1.37
+  // times the time, 1.10 by geometric mean), though they take 0.92 of it up to 500.
+  static constexpr int kWaves = D == 64 ? 8 : 4;
   static constexpr int kThreads = kWaves * kWave;
   static constexpr int kTile = 16;                          // positions of a key tile
   static constexpr int kStage = kTile * kWaves;             // positions of a stage
@@ -281,6 +283,9 @@ struct Geo {
   static constexpr int kWeights = 2 * kWaves * 2 * kTileBytes;
   static constexpr int kLds = kWeights + 2 * kWaves * RT * 512;
   static_assert(kLds + RT * kWaves * 128 + 256 <= (int)kMaxLds, "LDS budget");
+  // Wavefronts a SIMD: of one workgroup, or of two where LDS holds two.
+  static constexpr int kMinOnSimd = kWaves / 4;
+  static constexpr int kMaxOnSimd = kWaves == 4 && 2 * (kLds + RT * kWaves * 64 + 64) <= (int)kMaxLds ? 2 : kWaves / 4;
   // The 16-byte piece of row n that lands at LDS position p is piece p ^ swz(n): 16 consecutive rows
   // read at one piece index then hit 16 distinct bank groups.
   __device__ static __forceinline__ int swz(int n) { return kChunks >= 16 ? (n & 15) : ((n >> 1) & 7); }
@@ -291,7 +296,7 @@ struct Geo {
 // of branches, so that the compiler can count the vector-memory instructions outstanding.
 template <int D, int RT, bool ALIGNED>
 __global__ __launch_bounds__((Geo<D, RT>::kThreads))
-__attribute__((amdgpu_waves_per_eu((Geo<D, RT>::kWaves / 4), (Geo<D, RT>::kWaves / 4)))) void
+__attribute__((amdgpu_waves_per_eu((Geo<D, RT>::kMinOnSimd), (Geo<D, RT>::kMaxOnSimd)))) void
 spec_prefix_kernel(AttnArgs a) {
   using Gm = Geo<D, RT>;
   constexpr int kWaves = Gm::kWaves;

@@ -22,9 +22,12 @@ LOG2E = 1.4426950408889634
 # Defaults of the reference's call (spec_attn.py:136), except two sizes:
 # * num_splits: the reference fixes 64 (for an A100's 108 SMs); here None picks one prefix workgroup
 #   per compute unit, CUs // (num_reqs * num_kv_heads) splits (64 for one request with 4 kv heads on
-#   MI355X's 256 CUs).  A prefix workgroup holds a whole CU (over 128 KiB of LDS), so a grid larger than
-#   the CU count runs in two rounds.  A batch of 2 to 64 requests shares one such set of CUs //
-#   num_kv_heads slots by length (six requests of 9000 to 15700 positions: 46 -> 23 us a layer).
+#   MI355X's 256 CUs).  At D = 256 a prefix workgroup holds a whole CU (over 128 KiB of LDS), so a grid
+#   larger than the CU count runs in two rounds.  A batch of 2 to 64 requests shares one such set of
+#   CUs // num_kv_heads slots by length (six requests of 2335 to 9000 positions: 46 -> 23 us a layer)
+#   where that is two or more slots a request; with fewer there is little to share out and finding the
+#   plan only costs (64 requests x 8 kv heads, one of 404 positions, D = 256: 36.5 us balanced, 22.6
+#   even; equal lengths 1.04 times the even time).
 # * min_chunk: 64 positions instead of 128, so that short contexts spread over more workgroups.
 # block_n / num_warps / num_stages / combine_warps are Triton launch knobs there; the HIP kernels
 # have fixed shapes and ignore them.
@@ -106,9 +109,12 @@ def gqa_packed_spec_attention(query, key_cache, value_cache, out, seq_lens, bloc
     L = AL.load()
     attention, sets = L.qf_spec_attention, B
     if num_splits is None:
-        if 1 < B <= AL.MAX_BALANCED:  # one set of split slots a kv head, given out to the requests by length
+        num_splits = auto_num_splits(query.device, 1, num_kv_heads)
+        if 1 < B <= AL.MAX_BALANCED and num_splits >= 2 * B:
+            # one set of split slots a kv head, given out to the requests by length
             attention, sets = L.qf_spec_attention_balanced, 1
-        num_splits = max(B if sets == 1 else 1, auto_num_splits(query.device, sets, num_kv_heads))
+        else:
+            num_splits = auto_num_splits(query.device, B, num_kv_heads)
     ws_bytes = AL.workspace_bytes(sets, Q, H, num_kv_heads, D, num_splits)
     if ws_bytes == 0:
         raise ValueError("invalid attention sizes")

@@ -131,6 +131,28 @@ def test_balanced_batches(D, HKV, G, Q, page, lens):
     _check(inp, out, f"balanced D={D} HKV={HKV} G={G} Q={Q} page={page} lens={lens[:7]}")
 
 
+def test_balanced_where_two_slots_a_request(monkeypatch):
+    """The default call shares out a batch's splits by length where a kv head has two or more slots a request, and splits
+    evenly otherwise (one request, more requests than that, an explicit split count)."""
+    import torch
+    from qwen_fastpath import _attn_lib as AL
+    lib, calls = AL.load(), []
+
+    class Spy:
+        def __getattr__(self, name):
+            if name.startswith("qf_spec_attention"):
+                calls.append(name)
+            return getattr(lib, name)
+
+    monkeypatch.setattr(AL, "load", lambda: Spy())
+    slots = torch.cuda.get_device_properties(0).multi_processor_count // 4
+    for B, kw, want in ((1, {}, False), (2, {}, True), (slots // 2, {}, True), (slots // 2 + 1, {}, False), (2, {"num_splits": 8}, False)):
+        inp = A.gen_spec_inputs(90, 2, B, H=4, HKV=4, D=64, page=16, seed=B, lens=[92 - b % 40 for b in range(B)])
+        calls.clear()
+        _check(inp, _run(inp, **kw), f"B={B} {kw}")
+        assert ("qf_spec_attention_balanced" in calls) is (want and B <= 64), (B, kw, calls)
+
+
 def test_rows_that_see_nothing_are_zero():
     inp = A.gen_spec_inputs(0, 4, 3, seed=5, lens=[1, 2, 4])
     out = _run(inp)

@@ -1681,15 +1681,17 @@ __global__ void __launch_bounds__(W * kWave) quantize_tiled_kernel(const uint16_
 // segments of 64 bytes; K = 17408: 53.1 us, R = 8 over 100).
 constexpr int kQuantTiledMaxK = 18432;
 constexpr int kQuantTiledMinRows = 1024;
+constexpr int quant_tiled_rows(int K) { return K <= 8192 ? 8 : 4; }                           // rows a workgroup
+constexpr int quant_tiled_cap(int K) { return K <= 5120 ? 5120 : K <= 8192 ? 8192 : kQuantTiledMaxK; }  // values it keeps
 template <bool HEAD>
 hipError_t launch_quantize_tiled(const uint16_t* x, int64_t ldx, int M, int K, int8_t* image, float* scale,
                                  hipStream_t st) {
   const int rows = (M + 15) / 16 * 16;
   constexpr int W = 8;
   const dim3 block(W * kWave);
-  if (K <= 5120)
+  if (quant_tiled_cap(K) == 5120)
     hipLaunchKernelGGL((quantize_tiled_kernel<8, W, 5, HEAD>), dim3(rows / 8), block, 0, st, x, ldx, K, image, scale, M);
-  else if (K <= 8192)
+  else if (quant_tiled_cap(K) == 8192)
     hipLaunchKernelGGL((quantize_tiled_kernel<8, W, 8, HEAD>), dim3(rows / 8), block, 0, st, x, ldx, K, image, scale, M);
   else
     hipLaunchKernelGGL((quantize_tiled_kernel<4, W, 9, HEAD>), dim3(rows / 4), block, 0, st, x, ldx, K, image, scale, M);
@@ -4224,16 +4226,30 @@ int qf_quantize_rows_int8_tiled(const uint16_t* w, int64_t ldw, int8_t* image, f
              : QF_ERR_HIP;
 }
 
+// Whether several rows of a tile a workgroup (quantize_tiled_kernel) beat a workgroup a row for M tokens of K values.
+// Few rows put too few of them in flight (M = 333: 4.6 against 4.1 us at K = 5120, 8.4 against 7.3 at 17408).  From
+// 1024, what counts is how full the kernel is: the last round of one workgroup a CU, times the share of a lane's
+// registers that the row uses.  320 shapes of 1024 to 8192 rows and K 512 to 18432, x and image rotating past the
+// last-level cache: past 0.55 of both (K <= 4096, whose rows are short: 0.64 of the round alone; K > 8192, which stores
+// 64-byte segments: 0.7 of both, or one round) it takes 0.90 of the time by geometric mean, 1.04 at worst (17408 at
+// 2048 rows 31.9 -> 26.9 us); elsewhere 1.05, up to 1.24 (8256 at 6144 rows 40.4 -> 50.2).
+static bool quantize_tokens_in_tiles(int M, int K) {
+  if (M < kQuantTiledMinRows || K > kQuantTiledMaxK) return false;
+  const int cus = device_cus();
+  const int wgs = round_up16(M) / quant_tiled_rows(K);
+  const double fill = (double)wgs / ((double)ceil_div(wgs, cus) * cus);
+  const double full = fill * K / quant_tiled_cap(K);
+  if (K > 8192) return full >= 0.7 || wgs <= cus;
+  return full >= 0.55 || (K <= 4096 && fill >= 0.64);
+}
+
 static int quantize_tokens(const uint16_t* x, int64_t ldx, int M, int K, int8_t* xq, int64_t ldq, float* s_a,
                            int tiled, void* stream) {
   if (x == nullptr || xq == nullptr || s_a == nullptr || M < 1 || K < 1 || ldx < K || ldq < K) return QF_ERR_INVALID_ARG;
   if (K % QF_W8A16_K_ALIGN || !aligned16(x) || ldx % 8 || (uintptr_t)xq % 8 || ldq % 8) return QF_ERR_UNSUPPORTED;
   if (tiled && !aligned16(xq)) return QF_ERR_UNSUPPORTED;
   const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  // Many rows: several rows of a tile a workgroup (whole lines stored); few: a workgroup a row, which
-  // puts more of them in flight (us, new against old: M = 333 4.6 / 4.1 at K = 5120 and 8.4 / 7.3 at 17408, M = 1024
-  // 5.6 / 5.6 and 13.4 / 17.4, M = 2048 8.3 / 11.3 and 26.1 / 29.7).
-  if (tiled && M >= kQuantTiledMinRows && K <= kQuantTiledMaxK)
+  if (tiled && quantize_tokens_in_tiles(M, K))
     return launch_quantize_tiled<false>(x, ldx, M, K, xq, s_a, st) == hipSuccess ? QF_OK : QF_ERR_HIP;
   const int per_thread = ceil_div(K / 8, 256);  // 16-byte pieces a thread
   const dim3 grid(tiled ? round_up16(M) : M);

@@ -4228,19 +4228,20 @@ int qf_quantize_rows_int8_tiled(const uint16_t* w, int64_t ldw, int8_t* image, f
 
 // Whether several rows of a tile a workgroup (quantize_tiled_kernel) beat a workgroup a row for M tokens of K values.
 // Few rows put too few of them in flight (M = 333: 4.6 against 4.1 us at K = 5120, 8.4 against 7.3 at 17408).  From
-// 1024, what counts is how full the kernel is: the last round of one workgroup a CU, times the share of a lane's
-// registers that the row uses.  320 shapes of 1024 to 8192 rows and K 512 to 18432, x and image rotating past the
-// last-level cache: past 0.55 of both (K <= 4096, whose rows are short: 0.64 of the round alone; K > 8192, which stores
-// 64-byte segments: 0.7 of both, or one round) it takes 0.90 of the time by geometric mean, 1.04 at worst (17408 at
-// 2048 rows 31.9 -> 26.9 us); elsewhere 1.05, up to 1.24 (8256 at 6144 rows 40.4 -> 50.2).
+// 1024, what counts is how full the last round of one workgroup a CU is, and the share of a lane's registers that a row
+// uses: `fill`, and both as `full`.  Against a workgroup a row, x and image rotating past the last-level cache, 322 shapes
+// of 1024 to 8192 rows and K 320 to 18432: where this rule takes it 0.91 of the time by geometric mean, at worst 1.06
+// (4096 rows of 5120 14.9 against 18.7 us), elsewhere 1.13, up to 1.41 (1024 rows of 5184 8.3 against 5.9); 160 other
+// shapes the same (1.03 at worst).
 static bool quantize_tokens_in_tiles(int M, int K) {
   if (M < kQuantTiledMinRows || K > kQuantTiledMaxK) return false;
   const int cus = device_cus();
   const int wgs = round_up16(M) / quant_tiled_rows(K);
   const double fill = (double)wgs / ((double)ceil_div(wgs, cus) * cus);
   const double full = fill * K / quant_tiled_cap(K);
-  if (K > 8192) return full >= 0.7 || wgs <= cus;
-  return full >= 0.55 || (K <= 4096 && fill >= 0.64);
+  if (K > 8192) return full >= 0.66 || (fill >= 0.8 && full >= 0.59);  // 64-byte segments: long rows only
+  if (wgs <= cus) return K >= 4096 && (fill >= 0.8 || (K > 6144 && full >= 0.59));
+  return fill >= (K < 3072 ? 0.8 : 0.66) && (K <= 5120 || full >= 0.66);
 }
 
 static int quantize_tokens(const uint16_t* x, int64_t ldx, int M, int K, int8_t* xq, int64_t ldq, float* s_a,

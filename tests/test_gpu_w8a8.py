@@ -448,8 +448,8 @@ def test_w8a8_tile_kernel_128_token_workgroups(M, N, K):
 
 @pytest.mark.parametrize("M,K", [(1, 64), (15, 128), (16, 1024), (17, 5120), (300, 8192), (2048, 5120),
                                  (33, 17408), (1023, 5120), (1024, 64), (1029, 5184), (1040, 8192), (1025, 8256),
-                                 (1031, 18432), (1027, 18496), (2041, 64), (2033, 5120), (2047, 5184), (2046, 8192),
-                                 (1024, 8256), (2039, 13824), (2035, 18432)])
+                                 (1031, 18432), (1027, 18496), (4081, 64), (2033, 5120), (2047, 5184), (2046, 8192),
+                                 (4090, 5568), (2039, 13824), (1024, 11200), (2035, 18432)])
 def test_quantize_tokens_tiled_image(M, K):
     """qf_quantize_tokens_int8_tiled writes the same scales as the row-major quantiser and, byte for byte,
     the token-tiled image of its xq (rows past M zero), over a buffer that starts filled with garbage."""

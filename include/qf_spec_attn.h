@@ -86,10 +86,11 @@ int qf_spec_attention(const uint16_t* query, int64_t q_stride_tok, int64_t q_str
 
 /* qf_spec_attention with one set of split slots per kv head shared by all requests: total_splits slots
  * (num_reqs <= total_splits <= 65535, num_reqs <= 64, else QF_ERR_UNSUPPORTED) are given out by length, one
- * chunk length for the whole batch (at least min_chunk, a multiple of QF_SPEC_ATTN_KEY_BLOCK), so a ragged
- * batch's longest split is about its mean.  Workspace: qf_spec_attn_workspace_bytes(1, q_len, num_heads,
- * num_kv_heads, head_size, total_splits) + QF_SPEC_ATTN_PLAN_BYTES.  The rest as qf_spec_attention; the results differ by the order of
- * the fp32 sums only.  No reference counterpart (the reference splits every request num_splits ways,
+ * chunk length for the whole batch (at least min_chunk, a multiple of QF_SPEC_ATTN_KEY_BLOCK, found in steps
+ * of an eighth), so a ragged batch's longest split is near its mean and not the longest request's share.
+ * Workspace: qf_spec_attn_workspace_bytes(1, q_len, num_heads, num_kv_heads, head_size, total_splits) +
+ * QF_SPEC_ATTN_PLAN_BYTES.  The rest as qf_spec_attention; the results differ by where a request is cut: the
+ * order of the fp32 sums and the reference against which a softmax weight is rounded.  No reference counterpart (the reference splits every request num_splits ways,
  * plugin/qwen_fastpath/spec_attn.py:38-40). */
 int qf_spec_attention_balanced(const uint16_t* query, int64_t q_stride_tok, int64_t q_stride_head,
                                const uint16_t* key_cache, int64_t k_stride_block, int64_t k_stride_tok,

@@ -131,6 +131,43 @@ def test_balanced_batches(D, HKV, G, Q, page, lens):
     _check(inp, out, f"balanced D={D} HKV={HKV} G={G} Q={Q} page={page} lens={lens[:7]}")
 
 
+def _growing_poisoned(lens, Q, D, HKV, G, page, seed):
+    """A batch whose later positions score higher, so that the exponent references move in stage after stage, and the same
+    cache with NaN in every row that no query may see."""
+    inp = A.gen_spec_inputs(max(lens), Q, len(lens), H=G * HKV, HKV=HKV, D=D, page=page, seed=seed, lens=lens)
+    unseen = np.ones(inp.kv.shape[:1] + inp.kv.shape[2:3], dtype=bool)  # [page id, row]
+    for b, n in enumerate(lens):
+        pos = np.arange(n)
+        blk, off = inp.block_table[b, pos // page], pos % page
+        unseen[blk, off] = False
+        k = A.bf16_bits_to_f32(inp.kv[blk, :, off, :D]) * (1.0 + 6.0 * pos / n)[:, None, None]
+        inp.kv[blk, :, off, :D] = A.bf16_bits_from_f32(k.astype(np.float32))
+    poisoned = inp.kv.copy()
+    poisoned.transpose(0, 2, 1, 3)[unseen] = 0x7FC0
+    return inp, poisoned
+
+
+@pytest.mark.parametrize("D,G,Q,page,lens", [
+    # 8 wavefronts, 128 positions a stage, wavefronts in two row groups
+    (64, 8, 2, 17, [700, 643]), (64, 8, 3, 64, [900, 517]), (64, 8, 3, 24, [900, 517]),
+    (64, 8, 5, 64, [1100, 641]), (64, 8, 5, 17, [1100, 641]), (64, 8, 8, 16, [1300, 650]), (64, 7, 8, 24, [1300, 650]),
+    # 4 wavefronts, 64 positions a stage
+    (128, 4, 3, 17, [600, 449]), (128, 8, 5, 24, [600, 449]), (128, 8, 8, 17, [600, 449]),
+    (256, 6, 2, 24, [600, 449]), (256, 6, 3, 17, [600, 449]), (256, 8, 8, 24, [600, 449]),
+    # more than 64 stages: the block ids are read again
+    (256, 6, 3, 17, [4500]), (128, 2, 4, 24, [4460]), (64, 2, 2, 17, [8600]), (64, 2, 2, 32, [8600]),
+])
+def test_long_splits(D, G, Q, page, lens):
+    """One split a request, several stages long, on pages that hold whole key tiles and pages that cut them."""
+    inp, poisoned = _growing_poisoned(lens, Q, D, 2, G, page, seed=D + G + Q + page)
+    clean = inp.kv
+    for kw in ({"num_splits": 1}, {"min_chunk": 1 << 20}):
+        inp.kv = poisoned
+        out = _run(inp, **kw)
+        inp.kv = clean
+        _check(inp, out, f"long splits D={D} G={G} Q={Q} page={page} lens={lens} {kw}")
+
+
 def test_balanced_where_two_slots_a_request(monkeypatch):
     """The default call shares out a batch's splits by length where a kv head has two or more slots a request, and splits
     evenly otherwise (one request, more requests than that, an explicit split count)."""

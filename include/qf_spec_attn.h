@@ -90,8 +90,8 @@ int qf_spec_attention(const uint16_t* query, int64_t q_stride_tok, int64_t q_str
  * of an eighth), so a ragged batch's longest split is near its mean and not the longest request's share.
  * Workspace: qf_spec_attn_workspace_bytes(1, q_len, num_heads, num_kv_heads, head_size, total_splits) +
  * QF_SPEC_ATTN_PLAN_BYTES.  The rest as qf_spec_attention; the results differ by where a request is cut: the
- * order of the fp32 sums and the reference against which a softmax weight is rounded.  No reference counterpart (the reference splits every request num_splits ways,
- * plugin/qwen_fastpath/spec_attn.py:38-40). */
+ * order of the fp32 sums and the exponent reference against which a softmax weight is rounded.  No reference
+ * counterpart (the reference splits every request num_splits ways, plugin/qwen_fastpath/spec_attn.py:38-40). */
 int qf_spec_attention_balanced(const uint16_t* query, int64_t q_stride_tok, int64_t q_stride_head,
                                const uint16_t* key_cache, int64_t k_stride_block, int64_t k_stride_tok,
                                int64_t k_stride_head,

@@ -188,11 +188,11 @@ int qf_w8a16_gemm_noalloc(const uint16_t* x, int64_t ldx,
  * address or memory channel takes many of the atomics), and a second launch of one wavefront per token
  * folds the slots into the ids and clears them.
  * Served where the MFMA kernel would run without a K split (else QF_ERR_UNSUPPORTED: call qf_w8a16_gemm
- * and qf_argmax_rows_bf16); an automatic call runs the kernel that qf_w8a16_gemm runs there.  Workspace: qf_w8a16_argmax_workspace_bytes() bytes with the
- * split-K workspace contract: its first QF_W8A16_COUNTER_BYTES bytes (the slots) must be zero when a
- * call starts and are zero again when it ends, so a workspace zeroed once serves any number of calls
- * issued in order on one stream (a split-K workspace may serve); calls that may run at the same time
- * need distinct workspaces.  1 <= n_valid <= N.
+ * and qf_argmax_rows_bf16); an automatic call runs the kernel that qf_w8a16_gemm runs there.
+ * Workspace: qf_w8a16_argmax_workspace_bytes() bytes with the split-K workspace contract: its first
+ * QF_W8A16_COUNTER_BYTES bytes (the slots) must be zero when a call starts and are zero again when it ends,
+ * so a workspace zeroed once serves any number of calls issued in order on one stream (a split-K workspace
+ * may serve); calls that may run at the same time need distinct workspaces.  1 <= n_valid <= N.
  * Reference: the W8A16 logits and the pad-masked argmax of get_top_tokens,
  * plugin/qwen_fastpath/patches.py:160-166,178-185, in one launch. */
 int qf_w8a16_gemm_argmax(const uint16_t* x, int64_t ldx, const int8_t* w, int64_t ldw, int layout,

@@ -125,11 +125,12 @@ __device__ __forceinline__ int wave_scan(int v) {
 
 // The balanced split (every lane of the wavefront active; at most kMaxBalanced requests, splits >= requests): one
 // chunk length for all requests, the shortest of a rising sequence of multiples of kKeyBlock whose splits fit the
-// a.splits slots of a kv head (each candidate an eighth above the last), so the longest split of a ragged batch is near
-// the batch's mean and not the longest request's share (six requests of 9000 to 2335 positions: 640 positions, 55 of 64
-// slots used, the mean 531).  A request without a prefix takes one split (its in-flight positions).  Slots go to the requests
-// in order.  Lane i returns request i's length, splits (n) and first slot; `total` slots are used.  In unsigned
-// arithmetic and in units of kKeyBlock, so that min_chunk may be any int and the batch hold up to 2^36 positions.
+// a.splits slots of a kv head (each candidate an eighth above the last), so the longest split of a ragged batch is
+// near the batch's mean and not the longest request's share (six requests of 9000 to 2335 positions: 640 positions,
+// 55 of 64 slots used, the mean 531).  A request without a prefix takes one split (its in-flight positions).  Slots
+// go to the requests in order.  Lane i returns request i's length, splits (n) and first slot; `total` slots are used.
+// In unsigned arithmetic and in units of kKeyBlock, so that min_chunk may be any int and the batch hold up to 2^36
+// positions.
 __device__ __forceinline__ void balance(const AttnArgs& a, int lane, int& seq, int& chunk, int& n, int& first, int& total) {
   seq = lane < a.B ? a.seq_lens[lane] : 0;
   const uint32_t prefix = (uint32_t)max(seq - a.Q, 0);
@@ -647,12 +648,11 @@ spec_prefix_kernel(AttnArgs a) {
   }
 }
 
-// One workgroup per (token, head, 64-wide slice of d): the row's split partials merged by log-sum-exp
-// (the merge of the reference's _suffix_combine_kernel, spec_attn.py:119-131).  Every split has
-// written its rows' log-sum-exp (-inf where it saw nothing), so all loads issue at once, with no
-// dependence on the sequence length (balanced calls read the request's place among the slots first);
-// 16 groups of 16 threads merge every 16th split, then LDS merges
-// the groups.
+// One workgroup per (token, head, 64-wide slice of d): the row's split partials merged by log-sum-exp (the merge of
+// the reference's _suffix_combine_kernel, spec_attn.py:119-131).  Every split has written its rows' log-sum-exp (-inf
+// where it saw nothing), so all loads issue at once, with no dependence on the sequence length (balanced calls read
+// the request's place among the slots first); 16 groups of 16 threads merge every 16th split, then LDS merges the
+// groups.
 constexpr int kCombSlice = 64;  // d values per combine workgroup
 
 template <int D>

@@ -1119,16 +1119,15 @@ __global__ void __launch_bounds__(W * kWave) w8a16_stream_xreg_kernel(const Gemm
 // wavefront (32 KiB a CU in flight) measured best of 2, 3, 4 and 6; the x requests go out before the weights (level
 // with after); 8-byte fragment granules, which halve the lines of an x request, are level too.
 // LINES: the rows start on 128-byte lines, so no line is read twice and the copies bypass reuse (non-temporal: gate_up
-// M = 11 32.5 against 35.8 us); rows that do not (K an odd number of steps) share each line between two wavefronts' pairs
+// M = 11 3 us faster); rows that do not (K an odd number of steps) share each line between two wavefronts' pairs
 // and keep it cached (N = 6539, K = 10944, M = 14: 22.2 against 23.0 us).
 // Sums in a fixed order as in the stream kernel: each wavefront parks its partial tile in LDS, wavefront v then adds
 // the 8 partials of tiles v, v + 8, ... in wavefront order; with a K split the last workgroup of a run adds the splits
 // in split order (the MFMA kernel's device-scope partials and arrival counter).
-// Bound by memory on wide weights (gate_up M = 5 31.2 us, 5.7 TB/s, against 43.0 on the MFMA kernel; M = 11 32.5
-// against 52.5; M = 16 34.0 against 49.9), by the x requests' L2 traffic, the run's unevenness and the sums on narrow
-// ones (M = 11: qkv 14.6 against 20.3, o_proj 13.8 against 15.2, down 22.8 against 24.7).  Over 90 shapes of 512 to
-// 40000 channels, K 512 to 17920 and M 2 to 16 drawn at random it takes 0.75 of the time of the kernels before it, at
-// worst 1.07 (an odd K whose pairs do not share out over the wavefronts).
+// Bound by memory on wide weights (gate_up M = 5 32.2 us, 5.5 TB/s, against 43.0 on the MFMA kernel; M = 11 33.5
+// against 52.4; M = 16 34.9 against 49.7), by the x requests' L2 traffic, the run's unevenness and the sums on narrow
+// ones (M = 5 / 11: qkv 13.4 / 14.8 against 16.4 / 20.1, o_proj 13.1 / 14.6 against 13.0 / 15.2, down 20.9 / 23.4 against
+// 22.3 / 24.8).  Random shapes: rows_lose_lines.
 // ---------------------------------------------------------------------------------------------
 constexpr int kRowsWaves = 8;
 constexpr int kRowsSlots = 2;
@@ -1614,17 +1613,17 @@ __global__ void __launch_bounds__(256) quantize_tokens_kernel(const uint16_t* x,
   }
 }
 
-// Per-row quantiser straight into the TILED image (HEAD: the draft head's rows, s = max(amax, 1e-8) fl(1/127),
-// clamp +-127; else tokens, s = amax fl(1/127), clamp [-128, 127]).  A workgroup of W wavefronts takes R rows of one
-// 16-row tile: lane (c, r) of a wavefront holds 16 consecutive values of row r (two 16-byte loads), which are exactly
-// one 16-byte piece of the image, and the R pieces at one k lie side by side there, so every store instruction writes
-// 64 / R segments of 16 R contiguous bytes (R = 16: one whole KiB, R = 8: whole 128-byte lines) and no line is put
-// together from several workgroups.  The row's values stay in registers between the maximum and the rounding (NP
-// piece pairs a lane).  Memory-bound: tokens
-// 4096 x 5120 / 8192 / 17408 (x rotating past the last-level cache) 14.5 / 22.0 / 53.1 us against 18.1 / 29.1 / 55.6
-// for a workgroup a row; the 151936 x 5120 head 411 us (5.7 TB/s) against 443 + 272 us for the quantiser and the
-// repack.  W = 16, R = 16 and R = 4 at K = 5120: 15.2 to 16.7 us, the head 423 to 483 us.  Non-temporal token loads
-// are 3% faster, non-temporal stores 5% more here, but the GEMM that reads the image then loses it (level together).
+// Per-row quantiser straight into the TILED image (HEAD: the draft head's rows, s = max(amax, 1e-8) fl(1/127), clamp
+// +-127; else tokens, s = amax fl(1/127), clamp [-128, 127]).  A workgroup of W wavefronts takes R rows of one 16-row
+// tile: lane (c, r) of a wavefront holds 16 consecutive values of row r (two 16-byte loads), which are exactly one
+// 16-byte piece of the image, and the R pieces at one k lie side by side there, so every store instruction writes 64
+// / R segments of 16 R contiguous bytes (R = 16: one whole KiB; R = 8: whole 128-byte lines, so that no line is put
+// together from several workgroups; R = 4: halves of them).  The row's values stay in registers between the maximum
+// and the rounding (NP piece pairs a lane).  Memory-bound: tokens 4096 x 5120 / 8192 / 17408 (x rotating past the
+// last-level cache) 14.5 / 22.0 / 53.1 us against 18.1 / 29.1 / 55.6 for a workgroup a row; the 151936 x 5120 head
+// 411 us (5.7 TB/s) against 443 + 272 us for the quantiser and the repack.  W = 16, R = 16 and R = 4 at K = 5120:
+// 15.2 to 16.7 us, the head 423 to 483 us.  Non-temporal token loads are 3% faster, non-temporal stores 5% more here,
+// but the GEMM that reads the image then loses it (level together).
 template <int R, int W, int NP, bool HEAD>
 __global__ void __launch_bounds__(W * kWave) quantize_tiled_kernel(const uint16_t* x, int64_t ldx, int K, int8_t* image,
                                                                    float* scale, int M) {
@@ -1916,6 +1915,9 @@ constexpr int kW8A8TileLds = kW8A8TileStages * kW8A8TileStageBytes;
 // 612.6 -> 594.0 us, M = 8192 1236 -> 1147; down M = 4096 305.1 -> 294.1; o_proj M = 4096 148.9 -> 144.4;
 // qkv M = 8192 359.5 -> 339.9.  At 12 blocks (M = 3072) both orders measure the same (460.4 and 460.7 on
 // gate_up), and up to 8 the plain order already covers 8 x 4.  Bands of 2, 3, 6 and 8 were within 2% of 4.
+// The line counts blocks of the shape that runs, so 128-token workgroups run in bands from M = 1537, where both orders
+// are level: the 128 x 128 second launch at M = 2048 0.99 to 1.00 of the plain order's time (gate_up, qkv), reduce 3 (an
+// explicit choice there) 0.92 to 1.00 on gate_up and 0.98 to 1.02 on qkv, o_proj and down, the same code twice 0.99 to 1.01.
 constexpr int kW8A8TileBand = 4;
 constexpr int kW8A8TileBandRows = 12;
 constexpr int kW8A8TileMaxSplit = 8;                      // K splits of the tile kernel (fused reduction)
@@ -3405,9 +3407,9 @@ struct RowsPlan {
 
 // The least time of the busiest wavefront, in pairs (tiles of a run times pairs a tile), over the splits up to max_split
 // (the planes that the caller's workspace holds) that run in one round of workgroups, one a CU, with a run's partial
-// tiles in LDS (15 tiles: up to 61440 channels; a larger vocabulary keeps the MFMA kernel);
-// a split costs about a pair and a half, its partials' round trip: qkv 10240 x 5120
-// at M = 5 3 x 5 unsplit 13.1 us, 5 x 3 in two splits 14.8; o_proj 5120 x 8192 2 x 8 unsplit 13.8, 3 x 4 in two 13.6.
+// tiles in LDS (15 tiles: up to 61440 channels; a larger vocabulary keeps the MFMA kernel).  A split costs about a pair
+// and a half, its partials' round trip (tiles x pairs at M = 5: qkv 10240 x 5120 3 x 5 unsplit 13.1 us, 5 x 3 in two
+// splits 14.8; o_proj 5120 x 8192 2 x 8 unsplit 13.8, 3 x 4 in two 13.6, which the plan takes).
 RowsPlan rows_plan(int N, int K, int max_split) {
   const int all_pairs = (K / kStepK + 1) / 2;
   const int ntiles = round_up16(N) / kTileN;
